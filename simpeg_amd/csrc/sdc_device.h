@@ -44,8 +44,9 @@ __device__ __forceinline__ uint32_t xcd_remap(uint32_t b, uint32_t nb) {
 
 // Coefficients of the 7-point nodal operator on one grid level.
 //   cx[n]: conductance of the +x edge of node n (0 on the last x node), same for cy, cz
-//   dg[n]: full diagonal sum(edge conductances) + Robin term
-//   idg[n]: 1/dg[n]
+//   rd[n]: rest of the diagonal: the Robin term, plus, next to a pinned node 0, the conductance
+//          of the edge to it (1 on the pinned node itself)
+//   idg[n]: 1 / full diagonal
 // pin0 = 1: node 0 is an identity row and column (Neumann gauge, symmetric form)
 // pin0 = 2: node 0 is an identity row only (the nonsymmetric reference operator)
 template <typename T>
@@ -53,7 +54,7 @@ struct Sten {
   const T* cx;
   const T* cy;
   const T* cz;
-  const T* dg;
+  const T* rd;
   const T* idg;
   uint32_t n1x, n1y, n1z, nN, plane;
   FastDiv fx, fy;
@@ -73,7 +74,7 @@ __device__ __forceinline__ Sten<T> sten_col(Sten<T> s, int c) {
     s.cx += o;
     s.cy += o;
     s.cz += o;
-    s.dg += o;
+    s.rd += o;
     s.idg += o;
   }
   return s;
@@ -81,6 +82,11 @@ __device__ __forceinline__ Sten<T> sten_col(Sten<T> s, int c) {
 
 // Per-node stencil data.  The neighbour indices of a missing neighbour (domain edge) are the
 // node itself and its weight is 0, so stencil loads need no branches and stay in bounds.
+// d is the rest of the diagonal: (A x)_n = d x_n + sum of w (x_n - x_nbr).  Summed over
+// differences, a field that varies slowly loses nothing to the cancellation of its diagonal
+// term against its neighbours': with the full diagonal rounded to fp32, A had a spurious Robin
+// term of 6e-8 of the diagonal on every node, which on large or Neumann meshes is as large as
+// the true one and kept the fp32 recursion from following the true residual.
 template <typename T>
 struct NodeC {
   T wxm, wxp, wym, wyp, wzm, wzp, d;
@@ -117,7 +123,10 @@ __device__ __forceinline__ NodeC<T> node_coef(const Sten<T>& s, uint32_t n) {
   c.wxm = bx * (T)(hxm && !(p1 && n == 1));
   c.wym = by * (T)(hym && !(p1 && n == s.n1x));
   c.wzm = bz * (T)(hzm && !(p1 && n == s.plane));
-  c.d = s.dg[n];
+  // rd of node 0's neighbours holds their edge to it, which pin0 = 2 keeps as an edge
+  const bool p2 = s.pin0 == 2;
+  c.d = s.rd[n] - bx * (T)(p2 && n == 1) - by * (T)(p2 && n == s.n1x) -
+        bz * (T)(p2 && n == s.plane);
   return c;
 }
 
@@ -143,14 +152,6 @@ __device__ __forceinline__ void st_once(T* p, T v) {
   __builtin_nontemporal_store(v, p);
 }
 
-// (A x)_n for one column (x points at the column base).
-template <typename T>
-__device__ __forceinline__ T stencil(const NodeC<T>& c, const T* __restrict__ x, uint32_t n) {
-  const T xc = x[n], xw = x[c.ixm], xe = x[c.ixp], xs = x[c.iym], xn = x[c.iyp], xb = x[c.izm],
-          xt = x[c.izp];
-  return c.d * xc - c.wxm * xw - c.wxp * xe - c.wym * xs - c.wyp * xn - c.wzm * xb - c.wzp * xt;
-}
-
 // Column c0 + r of a block, clamped to the last column: loads of columns past ncol read valid
 // memory and their results are discarded, so no load needs a branch.
 template <typename T>
@@ -161,8 +162,9 @@ __device__ __forceinline__ const T* col_ptr(const T* x, size_t ld, int c0, int r
 
 // (A x)_n for R columns starting at column c0.  All 7R loads are issued before the arithmetic
 // so that a wavefront keeps them in flight; the per-lane indices are shared by every column.
-// The block may be stored in a narrower type X (bf16) than the arithmetic type T.
-template <typename T, int R, typename X>
+// The block may be stored in a narrower type X (bf16) than the arithmetic type T.  NBR: the
+// weighted sum of the six neighbours instead.
+template <typename T, int R, bool NBR = false, typename X>
 __device__ __forceinline__ void stencil_cols(const NodeC<T>& c, const X* __restrict__ x, uint32_t n,
                                              size_t ld, int c0, int ncol, T (&xc)[R], T (&v)[R]) {
   T xw[R], xe[R], xs[R], xn[R], xb[R], xt[R];
@@ -179,8 +181,11 @@ __device__ __forceinline__ void stencil_cols(const NodeC<T>& c, const X* __restr
   }
 #pragma unroll
   for (int r = 0; r < R; ++r)
-    v[r] = c.d * xc[r] - c.wxm * xw[r] - c.wxp * xe[r] - c.wym * xs[r] - c.wyp * xn[r] -
-           c.wzm * xb[r] - c.wzp * xt[r];
+    v[r] = NBR ? c.wxm * xw[r] + c.wxp * xe[r] + c.wym * xs[r] + c.wyp * xn[r] +
+                     c.wzm * xb[r] + c.wzp * xt[r]
+               : c.d * xc[r] + c.wxm * (xc[r] - xw[r]) + c.wxp * (xc[r] - xe[r]) +
+                     c.wym * (xc[r] - xs[r]) + c.wyp * (xc[r] - xn[r]) +
+                     c.wzm * (xc[r] - xb[r]) + c.wzp * (xc[r] - xt[r]);
 }
 
 // Sum R per-thread doubles over the work-group and write one partial per

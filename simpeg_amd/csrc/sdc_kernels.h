@@ -260,11 +260,11 @@ __global__ __launch_bounds__(SDC_BLOCK) void k_smooth_pair(Sten<T> sa, const B* 
   if (done && ld_flag(done)) return;
   SDC_NODE_PROLOGUE_C(sa.nN, sa.remap, R * G)
   if (!live) return;
-  // A x1 = c0 * A' b with the neighbour weights scaled by their 1/diagonal
+  // A x1 = c0 * (b - sum of w_nbr b_nbr / diagonal_nbr): the neighbour weights scaled by their
+  // 1/diagonal, the node's own diagonal times its inverse being 1
   auto scaled = [&](const Sten<T>& s, T& g) {
     NodeC<T> c = node_coef(s, n);
     g = s.idg[n];
-    c.d *= g;
     c.wxm *= s.idg[c.ixm];
     c.wxp *= s.idg[c.ixp];
     c.wym *= s.idg[c.iym];
@@ -280,14 +280,14 @@ __global__ __launch_bounds__(SDC_BLOCK) void k_smooth_pair(Sten<T> sa, const B* 
     const int cg = c0 + q * R;
     if (cg >= ncol) break;
     if (G > 1 && q > 0 && set_changes(sa, cg, cg - R)) c = scaled(sten_col(sa, cg), g);
-    T bc[R], ab[R];
-    stencil_cols<T, R>(c, b, n, ld, cg, ncol, bc, ab);
+    T bc[R], nb[R];
+    stencil_cols<T, R, true>(c, b, n, ld, cg, ncol, bc, nb);
 #pragma unroll
     for (int r = 0; r < R; ++r) {
       if (cg + r < ncol) {
         const size_t o = (size_t)(cg + r) * ld + n;
         const T x1 = cz * g * bc[r];
-        const T r1 = bc[r] - cz * ab[r];
+        const T r1 = bc[r] - cz * (bc[r] - nb[r]);
         st_once(xout + o, (X)(x1 + c1 * x1 + c2 * g * r1));
       }
     }
@@ -1180,9 +1180,15 @@ __global__ __launch_bounds__(SDC_FIN_THREADS) void k_norm_decide(const double* _
 // After a fold: the ring is empty and u is written.  After a reliable update also: the true
 // residual per column from the fp64 residual's partials (orr = rmax = |q - A u|^2, active =
 // orr > tol^2 |q|^2), then the stop rules: the solve stops when no column is open (converged),
-// at the iteration limit, or when the largest true relative residual failed to halve since the
-// previous update (the fp32 recursion stalled; the caller continues in fp64).  At the stop the
-// control block is also written to hctl (pinned host memory, may be null) for the host to read.
+// at the iteration limit, or when the largest true relative residual fell more slowly since the
+// previous update than 2^-SDC_STALL_RATE per iteration (the caller continues in fp64).  At the
+// stop the control block is also written to hctl (pinned host memory, may be null) for the host
+// to read.
+// The rate: an fp64 iteration costs 2.5-3 mixed ones and gains about 2.8 octaves of residual
+// (10 decades in 12 iterations), so a mixed phase below a quarter of that is slower than fp64.
+// Ordinary models gain 2.2 to 3.7 octaves per mixed iteration, a block of contrast 1e3 1.5, one
+// of 1e4 0.2 (174 iterations on 2,550 nodes without this rule, 32 + 7 fp64 ones with it).
+#define SDC_STALL_RATE 0.66
 __global__ __launch_bounds__(SDC_FIN_THREADS) void k_true_after(const double* __restrict__ partial,
                                                                 uint32_t nbx,
                                                                 const double* __restrict__ qn2,
@@ -1256,7 +1262,8 @@ __global__ __launch_bounds__(SDC_FIN_THREADS) void k_true_after(const double* __
       reason = 1;
     else if (it >= maxit)
       reason = 2;
-    else if (m > 0.5 * ld_flag(dctl + SDC_DCTL_MPREV))
+    else if (m > ld_flag(dctl + SDC_DCTL_MPREV) *
+                     exp2(-SDC_STALL_RATE * (it - ld_flag(ctl + SDC_CTL_LAST))))
       reason = 3;
     if (reason) {
       ctl[SDC_CTL_REASON] = reason;
@@ -1668,7 +1675,7 @@ struct Coef32 {
   float* cx;
   float* cy;
   float* cz;
-  float* dg;
+  float* rd;
   float* idg;
 };
 
@@ -1678,7 +1685,7 @@ struct DiagLevel {
   uint32_t n1x, n1y, nN, blk0;
   FastDiv fx, fy;
   const double *cx, *cy, *cz, *bd;
-  double *dg, *idg;
+  double *rd, *idg;
   size_t stride;
   Coef32 c32;
   int pin;
@@ -1689,9 +1696,10 @@ struct DiagLevels {
   int n;
 };
 
-// Full diagonal and its inverse of up to SDC_DIAG_LEVELS levels in one launch (work-groups
-// [lv[l].blk0, lv[l+1].blk0) take level l, blockIdx.z the operator set); with c32.cx set, also
-// the fp32 copies of cx, cy, cz, dg, idg (the fp32 solver's operator) in the same pass.
+// Rest of the diagonal (Sten::rd) and the inverse of the full one of up to SDC_DIAG_LEVELS
+// levels in one launch (work-groups [lv[l].blk0, lv[l+1].blk0) take level l, blockIdx.z the
+// operator set); with c32.cx set, also the fp32 copies of cx, cy, cz, rd, idg (the fp32 solver's
+// operator) in the same pass.
 __global__ __launch_bounds__(SDC_BLOCK) void k_coef_diag(DiagLevels tab) {
   int l = 0;
   while (l + 1 < tab.n && blockIdx.x >= tab.lv[l + 1].blk0) ++l;
@@ -1707,18 +1715,24 @@ __global__ __launch_bounds__(SDC_BLOCK) void k_coef_diag(DiagLevels tab) {
   const uint32_t k = fdiv(r, v.fy);
   const uint32_t j = r - k * v.n1y;
   const uint32_t plane = v.n1x * v.n1y;
-  double d = cx[n] + cy[n] + cz[n] + v.bd[zo + n];
+  double rd = v.bd[zo + n];
+  double d = cx[n] + cy[n] + cz[n] + rd;
   if (i > 0) d += cx[n - 1];
   if (j > 0) d += cy[n - v.n1x];
   if (k > 0) d += cz[n - plane];
-  if (v.pin && n == 0) d = 1.0;
-  v.dg[zo + n] = d;
+  if (v.pin) {
+    if (n == 0) rd = d = 1.0;
+    if (n == 1) rd += cx[0];
+    if (n == v.n1x) rd += cy[0];
+    if (n == plane) rd += cz[0];
+  }
+  v.rd[zo + n] = rd;
   v.idg[zo + n] = 1.0 / d;
   if (v.c32.cx) {
     v.c32.cx[zo + n] = (float)cx[n];
     v.c32.cy[zo + n] = (float)cy[n];
     v.c32.cz[zo + n] = (float)cz[n];
-    v.c32.dg[zo + n] = (float)d;
+    v.c32.rd[zo + n] = (float)rd;
     v.c32.idg[zo + n] = (float)(1.0 / d);
   }
 }
@@ -1867,7 +1881,7 @@ __global__ __launch_bounds__(1024) void k_coarse_inverse(Sten<double> s, double*
   s.cx += zo;
   s.cy += zo;
   s.cz += zo;
-  s.dg += zo;
+  s.rd += zo;
   s.idg += zo;
   inv64 += (size_t)blockIdx.x * astride;
   inv32 += (size_t)blockIdx.x * astride;
@@ -1881,7 +1895,7 @@ __global__ __launch_bounds__(1024) void k_coarse_inverse(Sten<double> s, double*
     double* row = a + (size_t)n * N;
     for (int m = 0; m < N; ++m) row[m] = 0.0;
     const NodeC<double> c = node_coef(s, (uint32_t)n);
-    row[n] = c.d;
+    row[n] = c.d + ((c.wxm + c.wxp) + (c.wym + c.wyp) + (c.wzm + c.wzp));
     if (c.ixm != (uint32_t)n) row[c.ixm] = -c.wxm;
     if (c.ixp != (uint32_t)n) row[c.ixp] = -c.wxp;
     if (c.iym != (uint32_t)n) row[c.iym] = -c.wym;

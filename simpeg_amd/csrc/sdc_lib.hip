@@ -132,16 +132,16 @@ struct Level {
   size_t ld = 0;
   // coefficient arrays hold one operator per set, sstride entries apart (round_ld(nN))
   size_t sstride = 0;
-  double *cx64 = nullptr, *cy64 = nullptr, *cz64 = nullptr, *bd64 = nullptr, *dg64 = nullptr,
+  double *cx64 = nullptr, *cy64 = nullptr, *cz64 = nullptr, *bd64 = nullptr, *rd64 = nullptr,
          *idg64 = nullptr;
-  float *cx32 = nullptr, *cy32 = nullptr, *cz32 = nullptr, *dg32 = nullptr, *idg32 = nullptr;
+  float *cx32 = nullptr, *cy32 = nullptr, *cz32 = nullptr, *rd32 = nullptr, *idg32 = nullptr;
   // transfer from this level to the next coarser one
   bool has_coarse = false;
   XferDev<double> x64;
   XferDev<float> x32;
   void release() {
-    dfree(cx64); dfree(cy64); dfree(cz64); dfree(bd64); dfree(dg64); dfree(idg64);
-    dfree(cx32); dfree(cy32); dfree(cz32); dfree(dg32); dfree(idg32);
+    dfree(cx64); dfree(cy64); dfree(cz64); dfree(bd64); dfree(rd64); dfree(idg64);
+    dfree(cx32); dfree(cy32); dfree(cz32); dfree(rd32); dfree(idg32);
     x64.release();
     x32.release();
   }
@@ -239,7 +239,7 @@ struct sdc_handle_s {
   int cset_cap = 0;
   const int32_t* cur_cset = nullptr;
   // scratch coefficient arrays for A(dsigma) (Jvec right-hand side)
-  double *tcx = nullptr, *tcy = nullptr, *tcz = nullptr, *tbd = nullptr, *tdg = nullptr,
+  double *tcx = nullptr, *tcy = nullptr, *tcz = nullptr, *tbd = nullptr, *trd = nullptr,
          *tidg = nullptr;
   // per-column-group partial sums of the adjoint contraction (jpart_cap doubles)
   double* jpart = nullptr;
@@ -248,6 +248,7 @@ struct sdc_handle_s {
   // a mixed solve stalled on the current operator and parameters: later mixed solves run fp64
   bool mixed_stalled = false;
   sdc_params prm;
+  int vstore = 1;  // storage of the fp32 V-cycle vectors in this call (as sdc_params.vcycle_bf16)
   int wlevel = 0;  // level whose coarse correction runs twice (0: none)
   int tail_level = 0;    // first level of the single-launch coarse tail (0: none)
   size_t tail_lds = 0;   // its LDS bytes per work-group
@@ -372,7 +373,7 @@ template <>
 Sten<double> make_sten<double>(const sdc_handle_s* h, int l, int pin_mode) {
   const Level& v = h->L[l];
   Sten<double> s{};
-  s.cx = v.cx64; s.cy = v.cy64; s.cz = v.cz64; s.dg = v.dg64; s.idg = v.idg64;
+  s.cx = v.cx64; s.cy = v.cy64; s.cz = v.cz64; s.rd = v.rd64; s.idg = v.idg64;
   s.n1x = v.n1x; s.n1y = v.n1y; s.n1z = v.n1z; s.nN = v.nN; s.plane = v.plane;
   s.fx = make_fastdiv(v.n1x); s.fy = make_fastdiv(v.n1y);
   s.pin0 = (h->bc == SDC_BC_NEUMANN) ? pin_mode : 0;
@@ -386,7 +387,7 @@ template <>
 Sten<float> make_sten<float>(const sdc_handle_s* h, int l, int pin_mode) {
   const Level& v = h->L[l];
   Sten<float> s{};
-  s.cx = v.cx32; s.cy = v.cy32; s.cz = v.cz32; s.dg = v.dg32; s.idg = v.idg32;
+  s.cx = v.cx32; s.cy = v.cy32; s.cz = v.cz32; s.rd = v.rd32; s.idg = v.idg32;
   s.n1x = v.n1x; s.n1y = v.n1y; s.n1z = v.n1z; s.nN = v.nN; s.plane = v.plane;
   s.fx = make_fastdiv(v.n1x); s.fy = make_fastdiv(v.n1y);
   s.pin0 = (h->bc == SDC_BC_NEUMANN) ? pin_mode : 0;
@@ -475,8 +476,8 @@ void fill_level_dims(Level& v) {
 }
 
 void free_level_arrays(Level& v) {
-  dfree(v.cx64); dfree(v.cy64); dfree(v.cz64); dfree(v.bd64); dfree(v.dg64); dfree(v.idg64);
-  dfree(v.cx32); dfree(v.cy32); dfree(v.cz32); dfree(v.dg32); dfree(v.idg32);
+  dfree(v.cx64); dfree(v.cy64); dfree(v.cz64); dfree(v.bd64); dfree(v.rd64); dfree(v.idg64);
+  dfree(v.cx32); dfree(v.cy32); dfree(v.cz32); dfree(v.rd32); dfree(v.idg32);
 }
 
 int alloc_level_arrays(Level& v, int nset) {
@@ -484,9 +485,9 @@ int alloc_level_arrays(Level& v, int nset) {
   v.sstride = round_ld(v.nN);
   const size_t n = v.sstride * (size_t)nset;
   CK(dmalloc(&v.cx64, n)); CK(dmalloc(&v.cy64, n)); CK(dmalloc(&v.cz64, n));
-  CK(dmalloc(&v.bd64, n)); CK(dmalloc(&v.dg64, n)); CK(dmalloc(&v.idg64, n));
+  CK(dmalloc(&v.bd64, n)); CK(dmalloc(&v.rd64, n)); CK(dmalloc(&v.idg64, n));
   CK(dmalloc(&v.cx32, n)); CK(dmalloc(&v.cy32, n)); CK(dmalloc(&v.cz32, n));
-  CK(dmalloc(&v.dg32, n)); CK(dmalloc(&v.idg32, n));
+  CK(dmalloc(&v.rd32, n)); CK(dmalloc(&v.idg32, n));
   return SDC_OK;
 }
 
@@ -555,10 +556,20 @@ Work<float>& work_of<float>(sdc_handle_s* h) { return h->w32; }
 template <>
 Work<double>& work_of<double>(sdc_handle_s* h) { return h->w64; }
 
+// Storage of the mixed solver's V-cycle vectors: sdc_params.vcycle_bf16, but fp32 (0) for Neumann
+// operators.  A pinned Neumann operator's smoothest mode is held by one node alone, so its energy
+// is below that of the rounding noise of a bf16 copy of it (2^-9 of each node's value, rough),
+// and PCG then removes that mode a little at a time: 104 iterations and an fp64 continuation
+// against 12 iterations with fp32 vectors on 54,600 nodes x 27 columns (28.5 against 3.4 ms), 100
+// against 14 on 667,680 x 28 (94 against 13 ms).
+int mixed_storage(const sdc_handle_s* h) {
+  return h->bc == SDC_BC_NEUMANN ? 0 : h->prm.vcycle_bf16;
+}
+
 // bytes per entry of the V-cycle vectors of the solver in precision T
 template <typename T>
 int vcycle_bytes(const sdc_handle_s* h) {
-  return (std::is_same<T, float>::value && h->prm.vcycle_bf16) ? 2 : (int)sizeof(T);
+  return (std::is_same<T, float>::value && h->vstore) ? 2 : (int)sizeof(T);
 }
 
 template <typename T>
@@ -566,7 +577,7 @@ int ensure_work(sdc_handle_s* h, int ncol) {
   Work<T>& w = work_of<T>(h);
   const int vb = vcycle_bytes<T>(h);
   const bool want16 =
-      std::is_same<T, float>::value && (h->prm.vcycle_bf16 == 3 || h->prm.vcycle_bf16 == 4);
+      std::is_same<T, float>::value && (h->vstore == 3 || h->vstore == 4);
   if (w.ncap >= ncol && w.vbytes == vb && (w.r16 != nullptr) == want16) return SDC_OK;
   ncol = std::max(ncol, w.ncap);
   drop_graphs(h);
@@ -1024,8 +1035,8 @@ template <typename T>
 int vcycle0(sdc_handle_s* h, const T* b, T* x, int ncol, bool dot_out, const int* done,
             hipStream_t st) {
   if constexpr (std::is_same<T, float>::value) {
-    if (h->prm.vcycle_bf16) return vcycle<float, __bf16, float, float>(h, 0, b, x, ncol, dot_out,
-                                                                       done, st);
+    if (h->vstore)
+      return vcycle<float, __bf16, float, float>(h, 0, b, x, ncol, dot_out, done, st);
   }
   return vcycle<T, T, T, T>(h, 0, b, x, ncol, dot_out, done, st);
 }
@@ -1167,6 +1178,7 @@ int pcg(sdc_handle_s* h, T* x, int ncol, double tol, int maxit, const int* col_m
 // run without a host synchronisation -- as one recorded graph when sdc_params.graph is set.
 int pcg_reliable(sdc_handle_s* h, const double* q, double* u, int ncol, const sdc_solve_opts* o,
                  sdc_solve_stats& S, hipStream_t st) {
+  h->vstore = mixed_storage(h);
   CK(ensure_work<float>(h, ncol));
   Work<float>& W = h->w32;
   const Level& l0 = h->L[0];
@@ -1200,10 +1212,10 @@ int pcg_reliable(sdc_handle_s* h, const double* q, double* u, int ncol, const sd
   const double delta2 = h->prm.reliable_delta * h->prm.reliable_delta;
   const int maxit = o->max_iter;
   // Stall guard: a reliable update is forced after kStallWindow iterations without one, and the
-  // solve gives up (converged = 0, the caller continues in fp64) when an update fails to halve
-  // the largest true relative residual of the previous one.  This happens when the fp32
-  // recursion no longer tracks the true residual (conductivity contrasts of 1e4 and more).
-  constexpr int kStallWindow = 25;
+  // solve gives up (converged = 0, the caller continues in fp64) when an update finds the true
+  // residual falling too slowly (k_true_after).  This happens when the bf16 multigrid no longer
+  // preconditions the operator (conductivity contrasts of 1e4 and more).
+  constexpr int kStallWindow = 16;
   // the device writes the control block to h_ctl when it stops (d_ctl), and the host reads the
   // stop flag there after each block of iterations: cleared before the first launch
   ((int*)h->h_ctl)[SDC_CTL_STOP] = 0;
@@ -1211,9 +1223,9 @@ int pcg_reliable(sdc_handle_s* h, const double* q, double* u, int ncol, const sd
   // cleared: the first fold writes it (and its column padding) without reading it
   hipLaunchKernelGGL(k_mixed_init, dim3(nblk(l0.nN)), blk, 0, st, W.qmask, l0.nN, W.ctl, W.qu, q,
                      u, tol2, delta2, maxit, kStallWindow);
-  // vcycle_bf16 = 3, 4: the multigrid reads a bfloat16 copy of r, written with r
-  __bf16* const r16 =
-      ((h->prm.vcycle_bf16 == 3 || h->prm.vcycle_bf16 == 4) && h->L.size() > 1) ? W.r16 : nullptr;
+  // storage 3, 4: the multigrid reads a bfloat16 copy of r, written with r
+  const int vst = h->vstore;
+  __bf16* const r16 = ((vst == 3 || vst == 4) && h->L.size() > 1) ? W.r16 : nullptr;
   DISPATCH_R(R, hipLaunchKernelGGL((k_ir_residual<float, R, true>), g, blk, 0, st, s2, q,
                                    (const double*)u, W.r, l0.ld, ncol, pf, W.partial, W.qmask, r16,
                                    (const int*)nullptr, (const double* const*)nullptr));
@@ -1233,8 +1245,8 @@ int pcg_reliable(sdc_handle_s* h, const double* q, double* u, int ncol, const sd
     hipLaunchKernelGGL(k_zero<double>, dim3(nblk(len)), blk, 0, st, u, len);
     return SDC_OK;
   }
-  // vcycle_bf16 = 1, 4: the preconditioned residual z is bfloat16
-  const bool zb = (h->prm.vcycle_bf16 == 1 || h->prm.vcycle_bf16 == 4) && h->L.size() > 1;
+  // storage 1, 4: the preconditioned residual z is bfloat16
+  const bool zb = (vst == 1 || vst == 4) && h->L.size() > 1;
   __bf16* const z16 = (__bf16*)W.xb0;
   const int K = std::max(1, (int)h->prm.check_every);
   // Early exits after the stop flag only matter when several iterations run between two host
@@ -1571,7 +1583,7 @@ int sdc_create(const sdc_mesh_desc* d, sdc_handle* out) {
   if ((rc = alloc_coarse_inverse(h, 1))) return bail(rc);
   const size_t n0 = h->L[0].nN;
   if ((rc = dmalloc(&h->tcx, n0)) || (rc = dmalloc(&h->tcy, n0)) || (rc = dmalloc(&h->tcz, n0)) ||
-      (rc = dmalloc(&h->tbd, n0)) || (rc = dmalloc(&h->tdg, n0)) || (rc = dmalloc(&h->tidg, n0)))
+      (rc = dmalloc(&h->tbd, n0)) || (rc = dmalloc(&h->trd, n0)) || (rc = dmalloc(&h->tidg, n0)))
     return bail(rc);
   if (hipHostMalloc((void**)&h->h_flag, 4 * sizeof(int), hipHostMallocDefault) != hipSuccess) {
     h->h_flag = nullptr;
@@ -1610,7 +1622,7 @@ int sdc_destroy(sdc_handle h) {
   dfree(h->bxm); dfree(h->bxp); dfree(h->bym); dfree(h->byp); dfree(h->bzm); dfree(h->bzp);
   for (auto& v : h->L) v.release();
   dfree(h->ainv64); dfree(h->ainv32); dfree(h->gj_a); dfree(h->gj_f);
-  dfree(h->tcx); dfree(h->tcy); dfree(h->tcz); dfree(h->tbd); dfree(h->tdg); dfree(h->tidg);
+  dfree(h->tcx); dfree(h->tcy); dfree(h->tcz); dfree(h->tbd); dfree(h->trd); dfree(h->tidg);
   dfree(h->jpart);
   dfree(h->cset_dev);
   h->w32.release();
@@ -1747,9 +1759,9 @@ int build_levels(sdc_handle_s* h, hipStream_t st, int nset) {
     for (size_t l = l0; l < h->L.size() && tab.n < SDC_DIAG_LEVELS; ++l) {
       Level& v = h->L[l];
       tab.lv[tab.n++] = DiagLevel{v.n1x, v.n1y, v.nN, nb, make_fastdiv(v.n1x),
-                                  make_fastdiv(v.n1y), v.cx64, v.cy64, v.cz64, v.bd64, v.dg64,
+                                  make_fastdiv(v.n1y), v.cx64, v.cy64, v.cz64, v.bd64, v.rd64,
                                   v.idg64, v.sstride,
-                                  Coef32{v.cx32, v.cy32, v.cz32, v.dg32, v.idg32}, pin};
+                                  Coef32{v.cx32, v.cy32, v.cz32, v.rd32, v.idg32}, pin};
       nb += (uint32_t)nblk(v.nN);
     }
     hipLaunchKernelGGL(k_coef_diag, dim3(nb, 1, z), dim3(SDC_BLOCK), 0, st, tab);
@@ -1812,6 +1824,7 @@ int sdc_vcycle(sdc_handle h, int dtype, const void* b, void* z, int ncol, void* 
     CK(ensure_work<double>(h, ncol));
     CK(vcycle0<double>(h, (const double*)b, (double*)z, ncol, false, nullptr, st));
   } else if (dtype == SDC_F32) {
+    h->vstore = h->prm.vcycle_bf16;
     CK(ensure_work<float>(h, ncol));
     CK(vcycle0<float>(h, (const float*)b, (float*)z, ncol, false, nullptr, st));
   } else {
@@ -1926,6 +1939,7 @@ int sdc_solve(sdc_handle h, const double* q, double* u, int ncol, const sdc_solv
     CK(fp64_solve(&it));
     S.iters = it;
   } else {
+    h->vstore = h->prm.vcycle_bf16;
     CK(ensure_work<float>(h, ncol));
     Work<float>& W = h->w32;
     hipLaunchKernelGGL(k_zero<double>, dim3(nblk(len)), blk, 0, st, u, len);
@@ -2022,10 +2036,10 @@ int sdc_jvec_rhs(sdc_handle h, const double* dsig, const double* u, double* out,
   DiagLevels tab{};
   tab.n = 1;
   tab.lv[0] = DiagLevel{l0.n1x, l0.n1y, l0.nN, 0, make_fastdiv(l0.n1x), make_fastdiv(l0.n1y),
-                        h->tcx, h->tcy, h->tcz, h->tbd, h->tdg, h->tidg, 0, Coef32{}, 0};
+                        h->tcx, h->tcy, h->tcz, h->tbd, h->trd, h->tidg, 0, Coef32{}, 0};
   hipLaunchKernelGGL(k_coef_diag, dim3(nblk(l0.nN)), dim3(SDC_BLOCK), 0, st, tab);
   Sten<double> s{};
-  s.cx = h->tcx; s.cy = h->tcy; s.cz = h->tcz; s.dg = h->tdg; s.idg = h->tidg;
+  s.cx = h->tcx; s.cy = h->tcy; s.cz = h->tcz; s.rd = h->trd; s.idg = h->tidg;
   s.n1x = l0.n1x; s.n1y = l0.n1y; s.n1z = l0.n1z; s.nN = l0.nN; s.plane = l0.plane;
   s.fx = make_fastdiv(l0.n1x); s.fy = make_fastdiv(l0.n1y);
   s.pin0 = 0;

@@ -41,8 +41,10 @@ __device__ __forceinline__ float apply_at(const Sten<float>& s, const float* x, 
                                           float& idg) {
   const NodeC<float> c = node_coef(s, n);
   idg = s.idg[n];
-  return c.d * x[n] - c.wxm * x[c.ixm] - c.wxp * x[c.ixp] - c.wym * x[c.iym] -
-         c.wyp * x[c.iyp] - c.wzm * x[c.izm] - c.wzp * x[c.izp];
+  const float xc = x[n];
+  return c.d * xc + c.wxm * (xc - x[c.ixm]) + c.wxp * (xc - x[c.ixp]) +
+         c.wym * (xc - x[c.iym]) + c.wyp * (xc - x[c.iyp]) + c.wzm * (xc - x[c.izm]) +
+         c.wzp * (xc - x[c.izp]);
 }
 
 // Chebyshev smoothing on one level.  b, x: this level's rhs and iterate; y: scratch.  On entry
