@@ -137,6 +137,7 @@ struct Level {
   float *cx32 = nullptr, *cy32 = nullptr, *cz32 = nullptr, *rd32 = nullptr, *idg32 = nullptr;
   // transfer from this level to the next coarser one
   bool has_coarse = false;
+  std::vector<int> rfine[3];  // per axis: fine index of every coarse node
   XferDev<double> x64;
   XferDev<float> x32;
   void release() {
@@ -250,8 +251,15 @@ struct sdc_handle_s {
   sdc_params prm;
   int vstore = 1;  // storage of the fp32 V-cycle vectors in this call (as sdc_params.vcycle_bf16)
   int wlevel = 0;  // level whose coarse correction runs twice (0: none)
-  int tail_level = 0;    // first level of the single-launch coarse tail (0: none)
-  size_t tail_lds = 0;   // its LDS bytes per work-group
+  // single-launch coarse tail: its first level (-1: none), its descriptor, the operator image of
+  // every set (tail_img_cap floats) and the tables; tail_stale: the image does not belong to the
+  // current operator or plan (ensure_tail)
+  int tail_level = -1;
+  TailDesc tail{};
+  float *tail_img = nullptr, *tail_tab = nullptr;
+  size_t tail_img_cap = 0, tail_tab_cap = 0;
+  bool tail_stale = true;
+  bool tail_at0 = true;  // the plan may start at the finest level
   Work<float> w32;
   Work<double> w64;
   int* h_flag = nullptr;  // pinned host copy of the convergence flag
@@ -541,6 +549,7 @@ int make_transfer(Level& f, Level& c, std::vector<int> (&fidx)[3]) {
   // Pz over (coarse x, coarse y, fine z)
   const size_t nwx = f.nN, nwy = (size_t)c.n1x * f.n1y * f.n1z,
                nwz = (size_t)c.n1x * c.n1y * f.n1z;
+  for (int a = 0; a < 3; ++a) f.rfine[a] = ri[a];
   f.x64.wxs = f.x32.wxs = round_ld(nwx);
   f.x64.wys = f.x32.wys = round_ld(nwy);
   f.x64.wzs = f.x32.wzs = round_ld(nwz);
@@ -638,6 +647,11 @@ int ensure_work(sdc_handle_s* h, int ncol) {
   return SDC_OK;
 }
 
+// top-level nodes per work-item of the coarse tail
+int tail_npt(uint32_t nN) {
+  return nN <= 2 * SDC_TAIL_THREADS ? 2 : nN <= 4 * SDC_TAIL_THREADS ? 4 : 8;
+}
+
 // W-cycle level: the requested one, or (wcycle_level = -1) the first level with at most 1/4 of
 // the finest level's nodes (level 1 unless the first coarsening step only touched a small core
 // of a padded mesh) -- a second visit there costs ~15 % of a cycle and removes an iteration on
@@ -656,28 +670,230 @@ int pick_wlevel(const sdc_handle_s* h) {
   return (l >= 1 && l < nl - 1) ? l : 0;
 }
 
-// First level of the coarse tail that one work-group per column runs out of LDS: the finest
-// level below the W-cycle level whose remaining levels fit (rhs + solution per level + one shared
-// scratch vector, fp32) into 160 KB, with at least one level above the coarsest.
-void pick_tail(sdc_handle_s* h) {
-  h->tail_level = 0;
-  h->tail_lds = 0;
+// The coarse tail that one work-group per column runs (sdc_tail.h): from the first level with at
+// most SDC_TAIL_NODES nodes whose cycle fits into 160 KB of LDS on, with at least one level above
+// the coarsest.  The finest level may be that one, unless it reads a bf16 residual (storage 3,
+// 4) or smooths another number of steps than the coarser ones.  On the 22,050-node block model the tail then starts at the W level (6,348 nodes), which
+// took 14 launches before.
+// at0 = false keeps the finest level out as well (sdc_vcycle, whose finest level shows the storage
+// it was asked for).
+void pick_tail(sdc_handle_s* h, bool at0 = true) {
+  h->tail_level = -1;
+  h->tail_stale = true;
+  h->tail_at0 = at0;
   const int nl = (int)h->L.size();
   if (!h->prm.fused_tail) return;
-  for (int lt = std::max(1, h->wlevel + 1); lt < nl - 1; ++lt) {
-    if (nl - lt > SDC_TAIL_MAX) continue;
-    size_t words = 0, ymax = 0;
-    for (int l = lt; l < nl; ++l) {
-      words += 2 * (size_t)h->L[l].nN;
-      ymax = std::max(ymax, (size_t)h->L[l].nN);
+  const int first = !at0 || h->prm.vcycle_bf16 == 3 || h->prm.vcycle_bf16 == 4 ||
+                            (h->prm.nu_coarse > 0 && (h->prm.nu_coarse != h->prm.nu_pre ||
+                                                      h->prm.nu_coarse != h->prm.nu_post))
+                        ? 1
+                        : 0;
+  for (int lt = first; lt < nl - 1; ++lt) {
+    const int nlev = nl - lt;
+    if (nlev > SDC_TAIL_MAX || h->L[lt].nN > SDC_TAIL_NODES) continue;
+    TailDesc d{};
+    auto up4 = [](size_t n) { return (n + 3) / 4 * 4; };
+    // LDS: the image (lower levels' coefficients, weights of the transfers below the top one),
+    // the tables, then the vectors
+    size_t o = 0;
+    for (int k = 0; k < nlev; ++k) {
+      const Level& v = h->L[lt + k];
+      TailLev& t = d.lv[k];
+      t.nN = v.nN;
+      t.n1x = v.n1x;
+      t.plane = v.plane;
+      if (k > 0 && k < nlev - 1) {
+        t.coef = (uint32_t)o;
+        o += 7 * (size_t)v.nN;
+      }
     }
-    const size_t bytes = (words + ymax) * sizeof(float);
-    if (bytes <= 160 * 1024) {
-      h->tail_level = lt;
-      h->tail_lds = bytes;
-      return;
+    for (int k = 0; k < nlev - 1; ++k) {
+      const Level& f = h->L[lt + k];
+      const Level& c = h->L[lt + k + 1];
+      TailXf& x = d.xf[k];
+      x.fn1x = f.n1x; x.fplane = f.plane;
+      x.cn1x = c.n1x; x.cplane = c.plane; x.cN = c.nN;
+      x.ys = c.n1x * f.n1y;
+      x.nwx = f.nN;
+      x.nwy = c.n1x * f.n1y * f.n1z;
+      if (k > 0) {
+        x.w = (uint32_t)o;
+        o += (size_t)x.nwx + x.nwy + (size_t)c.n1x * c.n1y * f.n1z;
+      }
+    }
+    d.nimg = (uint32_t)up4(o);
+    o = d.nimg;
+    d.ntop = (uint32_t)up4(2 * (size_t)d.xf[0].cN);
+    for (int k = 1; k < nlev - 1; ++k) {
+      d.xf[k].tab = (uint32_t)o;
+      o += 2 * (size_t)d.xf[k].cN;
+    }
+    d.ntab = (uint32_t)(up4(o) - d.nimg);
+    o = up4(o);
+    for (int k = 0; k < nlev; ++k) {
+      TailLev& t = d.lv[k];
+      const size_t halo = t.plane;
+      if (k == 0) {
+        t.x = (uint32_t)(o + halo);
+        o += (size_t)tail_npt(t.nN) * SDC_TAIL_THREADS + 2 * halo;
+      } else {
+        t.b = (uint32_t)o;
+        t.x = (uint32_t)(o + t.nN + halo);
+        t.y = (uint32_t)(t.x + t.nN + 2 * halo);
+        o += 3 * (size_t)t.nN + 4 * halo;
+      }
+    }
+    d.nlds = (uint32_t)up4(o);
+    if ((size_t)d.nlds * sizeof(float) > 160 * 1024) continue;
+    const TailXf& x0 = d.xf[0];
+    d.imgs = 8 * (size_t)tail_npt(d.lv[0].nN) * SDC_TAIL_THREADS + d.nimg +
+             up4((size_t)(SDC_TAIL_WR + SDC_TAIL_WP) * x0.cN);
+    // the cycle: down to the W level once, its coarse correction twice (once without a W level)
+    const int w = h->wlevel >= lt && h->wlevel > 0 ? h->wlevel - lt : -1;
+    const int last = nlev - 1;
+    auto step = [&](TailOp op, int l) {
+      d.op[d.nop] = op;
+      d.lev[d.nop++] = (uint8_t)l;
+    };
+    for (int l = 0; l < w; ++l) {
+      step(TAIL_PRE, l);
+      step(TAIL_DOWN, l);
+    }
+    if (w >= 0) step(TAIL_PRE, w);
+    for (int gam = 0; gam < (w >= 0 ? 2 : 1); ++gam) {
+      if (w >= 0) step(TAIL_DOWN, w);
+      for (int l = w + 1; l < last; ++l) {
+        step(TAIL_PRE, l);
+        step(TAIL_DOWN, l);
+      }
+      step(TAIL_DENSE, last);
+      for (int l = last - 1; l > w; --l) {
+        step(TAIL_UP, l);
+        step(TAIL_POST, l);
+      }
+      if (w >= 0) {
+        step(TAIL_UP, w);
+        step(gam == 0 ? TAIL_MID : TAIL_POST, w);
+      }
+    }
+    for (int l = w - 1; l >= 0; --l) {
+      step(TAIL_UP, l);
+      step(TAIL_POST, l);
+    }
+    h->tail = d;
+    h->tail_level = lt;
+    return;
+  }
+}
+
+// Partial sums per column of the r.z product that the cycle of the solver in precision T leaves
+// in Work::partial.
+template <typename T>
+uint32_t dot_blocks(const sdc_handle_s* h) {
+  return std::is_same<T, float>::value && h->tail_level == 0 ? 1u : nblk(h->L[0].nN);
+}
+
+// The tail's operator image and tables on the device, for the current plan and operator sets.
+int ensure_tail(sdc_handle_s* h, hipStream_t st, bool at0 = true) {
+  if (h->tail_at0 != at0) {
+    drop_graphs(h);
+    pick_tail(h, at0);
+  }
+  if (h->tail_level < 0 || !h->tail_stale) return SDC_OK;
+  const int lt = h->tail_level, nlev = (int)h->L.size() - lt;
+  TailDesc& d = h->tail;
+  const size_t need = d.imgs * (size_t)h->nset_cap;
+  const size_t ntab = (size_t)d.ntop + d.ntab;
+  if (h->tail_img_cap < need || h->tail_tab_cap < ntab) {
+    HIPCK(hipStreamSynchronize(st));
+    drop_graphs(h);
+    dfree(h->tail_img);
+    dfree(h->tail_tab);
+    h->tail_img_cap = h->tail_tab_cap = 0;
+    CK(dmalloc(&h->tail_img, need));
+    CK(dmalloc(&h->tail_tab, ntab));
+    h->tail_img_cap = need;
+    h->tail_tab_cap = ntab;
+    d.tab = nullptr;
+  }
+  if (!d.tab) {  // a new plan (pick_tail clears d) or a new buffer
+    std::vector<uint2> tab;
+    for (int k = 0; k < nlev - 1; ++k) {
+      const Level& f = h->L[lt + k];
+      const Level& c = h->L[lt + k + 1];
+      // the fine neighbour at fine index fi + s lies between coarse nodes
+      auto between = [&](int a, uint32_t C, int s) -> uint32_t {
+        const std::vector<int>& r = f.rfine[a];
+        return s < 0 ? C > 0 && r[C - 1] < r[C] - 1 : C + 1 < r.size() && r[C + 1] > r[C] + 1;
+      };
+      for (uint32_t K = 0; K < c.n1z; ++K)
+        for (uint32_t J = 0; J < c.n1y; ++J)
+          for (uint32_t I = 0; I < c.n1x; ++I) {
+            const uint32_t i = (uint32_t)f.rfine[0][I], j = (uint32_t)f.rfine[1][J],
+                           kk = (uint32_t)f.rfine[2][K];
+            const uint32_t flags = between(0, I, -1) | between(0, I, 1) << 1 |
+                                   between(1, J, -1) << 2 | between(1, J, 1) << 3 |
+                                   between(2, K, -1) << 4 | between(2, K, 1) << 5;
+            tab.push_back(tail_table_entry(i + f.n1x * (j + f.n1y * kk), flags,
+                                           I + c.n1x * (j + f.n1y * kk),
+                                           I + c.n1x * (J + c.n1y * kk)));
+          }
+      if (k == 0) tab.resize(d.ntop / 2, uint2{0, 0});
+    }
+    tab.resize(ntab / 2, uint2{0, 0});
+    HIPCK(hipMemcpyAsync(h->tail_tab, tab.data(), ntab * sizeof(float), hipMemcpyHostToDevice, st));
+    HIPCK(hipStreamSynchronize(st));
+  }
+  TailPack p{};
+  p.rows = (uint32_t)(tail_npt(d.lv[0].nN) * SDC_TAIL_THREADS);
+  size_t nmax = p.rows;
+  p.nlev = nlev - 1;
+  p.img = h->tail_img;
+  p.imgs = d.imgs;
+  const uint32_t base = 8 * p.rows;
+  for (int k = 0; k < nlev - 1; ++k) {
+    p.s[k] = make_sten<float>(h, lt + k, 1);
+    p.coef[k] = k == 0 ? 0 : base + d.lv[k].coef;
+    nmax = std::max(nmax, (size_t)d.lv[k].nN);
+    // the transfer's weights: below the top level copied into the LDS image
+    const Level& f = h->L[lt + k];
+    const Level& c = h->L[lt + k + 1];
+    const XferDev<float>& x = f.x32;
+    uint32_t dst = base + d.xf[k].w;
+    for (int a = 0; a < 3; ++a) {
+      TailPack::W& w = p.w[p.nw++];
+      const bool opd = h->prm.interp != 0;
+      const uint32_t g0 = a == 0 ? f.n1x : c.n1x, g1 = a == 2 ? c.n1y : f.n1y;
+      w.n = g0 * g1 * f.n1z;
+      if (opd) {
+        w.src = a == 0 ? x.wx : a == 1 ? x.wy : x.wz;
+        w.stride = (uint32_t)(a == 0 ? x.wxs : a == 1 ? x.wys : x.wzs);
+        w.d0 = 1;
+        w.d1 = 0xffffffffu;
+      } else {
+        w.src = a == 0 ? x.pwx : a == 1 ? x.pwy : x.pwz;
+        w.stride = 0;
+        w.d0 = a == 0 ? 1 : a == 1 ? g0 : g0 * g1;
+        w.d1 = a == 0 ? g0 : a == 1 ? g1 : f.n1z;
+      }
+      w.dst = dst;
+      dst += w.n;
+      if (k > 0) nmax = std::max(nmax, (size_t)w.n);
     }
   }
+  p.tab = (const uint2*)h->tail_tab;
+  p.x0 = d.xf[0];
+  p.top = base + d.nimg;
+  hipLaunchKernelGGL(k_tail_pack, dim3(nblk(nmax), (uint32_t)(p.nlev + 1 + p.nw - 3), (uint32_t)h->nset),
+                     dim3(SDC_BLOCK), 0, st, p);
+  HIPCK(hipGetLastError());
+  d.img = h->tail_img;
+  d.tab = h->tail_tab;
+  d.ainv = h->ainv32;
+  d.astride = (uint32_t)h->astride;
+  d.nn = (int)h->L.back().nN;
+  h->tail_stale = false;
+  return SDC_OK;
 }
 
 // Columns per work-item of the stencil kernels: automatic = 4 (measured on MI355X: the
@@ -757,41 +973,32 @@ Cheb cheb_coefs(const sdc_params& p) {
   return c;
 }
 
-// The V-cycle of levels tail_level .. L-1 for every column in one launch (one work-group per
-// column, all vectors in LDS); b and x are the tail level's blocks.
-template <typename S>
-int tail_vcycle(sdc_handle_s* h, const S* b, S* x, int ncol, const int* done, hipStream_t st) {
-  const int nl = (int)h->L.size();
-  const int lt = h->tail_level;
-  TailDesc d{};
-  d.nlev = nl - lt;
-  uint32_t off = 0, ymax = 0;
-  for (int k = 0; k < d.nlev; ++k) {
-    const int l = lt + k;
-    d.lv[k].s = make_sten<float>(h, l, 1);
-    if (l < nl - 1) d.lv[k].t = make_xfer<float>(h, l);
-    d.lv[k].offB = off;
-    off += h->L[l].nN;
-    d.lv[k].offX = off;
-    off += h->L[l].nN;
-    ymax = std::max(ymax, h->L[l].nN);
-  }
-  d.offY = off;
-  d.ainv = h->ainv32;
-  d.nn = (int)h->L[nl - 1].nN;
+// The cycle of levels tail_level .. L-1 for every column in one launch (one work-group per
+// column); b and x are the tail level's blocks; partial non-null: one b.x per column.
+template <typename B, typename O>
+int tail_cycle(sdc_handle_s* h, const B* b, O* x, int ncol, double* partial, const int* done,
+               hipStream_t st) {
+  if (h->tail_stale) return fail(SDC_ERR_STATE, "internal: tail image");
+  TailDesc d = h->tail;
   d.cset = h->cur_cset;
-  d.astride = (uint32_t)h->astride;
-  d.nu_pre = h->prm.nu_coarse > 0 ? h->prm.nu_coarse : h->prm.nu_pre;
-  d.nu_post = h->prm.nu_coarse > 0 ? h->prm.nu_coarse : h->prm.nu_post;
+  // level 0 smooths nu_pre / nu_post steps, coarser levels nu_coarse where that is set; a tail
+  // that holds both has one count for all its levels only if they agree (pick_tail)
+  const bool top = h->tail_level == 0 || h->prm.nu_coarse <= 0;
+  d.nu_pre = top ? h->prm.nu_pre : h->prm.nu_coarse;
+  d.nu_post = top ? h->prm.nu_post : h->prm.nu_coarse;
+  d.nu_mid = h->prm.wcycle_smooth > 0 ? h->prm.wcycle_smooth : d.nu_post;
   const Cheb cc = cheb_coefs(h->prm);
   for (int k = 0; k < 16; ++k) {
     d.c1[k] = (float)cc.c1[k];
     d.c2[k] = (float)cc.c2[k];
   }
-  const size_t bytes = (size_t)(off + ymax) * sizeof(float);
-  if (bytes != h->tail_lds) return fail(SDC_ERR_STATE, "internal: tail LDS size");
-  launch(h, k_tail_vcycle<S>, dim3(ncol), dim3(1024), bytes, st, d, b, x, h->L[lt].ld,
-                     done);
+  const dim3 g((uint32_t)ncol), blk(SDC_TAIL_THREADS);
+  const size_t lds = (size_t)d.nlds * sizeof(float), ld = h->L[h->tail_level].ld;
+  switch (tail_npt(d.lv[0].nN)) {
+    case 2: launch(h, k_tail_cycle<B, O, 2>, g, blk, lds, st, d, b, x, ld, partial, done); break;
+    case 4: launch(h, k_tail_cycle<B, O, 4>, g, blk, lds, st, d, b, x, ld, partial, done); break;
+    default: launch(h, k_tail_cycle<B, O, 8>, g, blk, lds, st, d, b, x, ld, partial, done); break;
+  }
   HIPCK(hipGetLastError());
   return SDC_OK;
 }
@@ -808,9 +1015,10 @@ int vcycle(sdc_handle_s* h, int l, const B* b, O* x, int ncol, bool dot_out, con
   const int G_ = pick_g(h, ncol);
   const Level& lv = h->L[l];
   const int nl = (int)h->L.size();
-  if constexpr (std::is_same<T, float>::value && std::is_same<B, S>::value &&
-                std::is_same<O, S>::value) {
-    if (h->tail_level > 0 && l == h->tail_level) return tail_vcycle<S>(h, b, x, ncol, done, st);
+  if constexpr (std::is_same<T, float>::value &&
+                (std::is_same<B, float>::value || std::is_same<O, __bf16>::value)) {
+    if (l == h->tail_level)
+      return tail_cycle<B, O>(h, b, x, ncol, dot_out ? W.partial : (double*)nullptr, done, st);
   }
   if (l == nl - 1) {
     const T* ainv = (const T*)(std::is_same<T, float>::value ? (const void*)h->ainv32
@@ -1114,7 +1322,8 @@ int pcg(sdc_handle_s* h, T* x, int ncol, double tol, int maxit, const int* col_m
   CK(graph_run(h, W.r, W.z, ncol, 8 + (int)sizeof(T), st, [&](hipStream_t gs) {
     return vcycle0<T>(h, W.r, W.z, ncol, true, nullptr, gs);
   }));
-  hipLaunchKernelGGL(k_fin_beta, dim3(ncol), blk, 0, st, (const double*)W.partial, nbx, W.rz,
+  const uint32_t nbz = dot_blocks<T>(h);
+  hipLaunchKernelGGL(k_fin_beta, dim3(ncol), blk, 0, st, (const double*)W.partial, nbz, W.rz,
                      W.beta, (const int*)W.active, 1, (const int*)nullptr);
   hipLaunchKernelGGL((k_update_p4<T, true>), grid4(l0.nN, ncol), blk, 0, st, (const T*)W.z, W.p,
                      (const double*)W.beta, l0.ld, l0.nN, (const int*)nullptr);
@@ -1138,7 +1347,7 @@ int pcg(sdc_handle_s* h, T* x, int ncol, double tol, int maxit, const int* col_m
            (const double*)W.bn2, (const int*)W.ctl, W.rr, W.active, W.counters, done,
            (int*)nullptr);
     CK(vcycle0<T>(h, W.r, W.z, ncol, true, vdone, s2));
-    launch(h, k_fin_beta, dim3(ncol), blk, 0, s2, (const double*)W.partial, nbx, W.rz, W.beta,
+    launch(h, k_fin_beta, dim3(ncol), blk, 0, s2, (const double*)W.partial, nbz, W.rz, W.beta,
            (const int*)W.active, 0, vdone);
     prof_begin(h, SDC_PROF_UPDATE_P, s2);
     launch(h, k_update_p4<T, false>, grid4(l0.nN, ncol), blk, 0, s2, (const T*)W.z, W.p,
@@ -1180,6 +1389,7 @@ int pcg_reliable(sdc_handle_s* h, const double* q, double* u, int ncol, const sd
                  sdc_solve_stats& S, hipStream_t st) {
   h->vstore = mixed_storage(h);
   CK(ensure_work<float>(h, ncol));
+  CK(ensure_tail(h, st));
   Work<float>& W = h->w32;
   const Level& l0 = h->L[0];
   const int R = pick_r(h, ncol);
@@ -1285,7 +1495,8 @@ int pcg_reliable(sdc_handle_s* h, const double* q, double* u, int ncol, const sd
     else
       rc = vcycle0<float>(h, W.r, W.z, ncol, true, stop, s);
     CK(rc);
-    launch(h, k_fin_beta, dim3(ncol), blk, 0, s, (const double*)W.partial, nbx, W.rz, W.beta,
+    launch(h, k_fin_beta, dim3(ncol), blk, 0, s, (const double*)W.partial, dot_blocks<float>(h),
+           W.rz, W.beta,
            (const int*)W.active, first ? 1 : 0, stop);
     // the class covers the steady-state launches (the first one skips p, q and x)
     const int atag = first ? -1 : SDC_PROF_APPLY;
@@ -1419,6 +1630,7 @@ int ensure_sets(sdc_handle_s* h, int nset) {
   }
   CK(alloc_coarse_inverse(h, nset));
   h->nset_cap = nset;
+  h->tail_stale = true;
   h->sigma_set = false;
   return SDC_OK;
 }
@@ -1602,11 +1814,17 @@ int sdc_create(const sdc_mesh_desc* d, sdc_handle* out) {
   }
   // the fused coarse tail and the coarsest inverse may use all 160 KB of LDS (set once,
   // outside any graph capture)
-  if (hipFuncSetAttribute((const void*)k_tail_vcycle<__bf16>,
-                          hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024) != hipSuccess ||
-      hipFuncSetAttribute((const void*)k_tail_vcycle<float>,
-                          hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024) != hipSuccess ||
-      hipFuncSetAttribute((const void*)k_coarse_inverse<true>,
+  const void* const big_lds[] = {
+      (const void*)k_tail_cycle<float, float, 2>,   (const void*)k_tail_cycle<float, float, 4>,
+      (const void*)k_tail_cycle<float, float, 8>,   (const void*)k_tail_cycle<float, __bf16, 2>,
+      (const void*)k_tail_cycle<float, __bf16, 4>,  (const void*)k_tail_cycle<float, __bf16, 8>,
+      (const void*)k_tail_cycle<__bf16, __bf16, 2>, (const void*)k_tail_cycle<__bf16, __bf16, 4>,
+      (const void*)k_tail_cycle<__bf16, __bf16, 8>};
+  for (const void* k : big_lds)
+    if (hipFuncSetAttribute(k, hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024) !=
+        hipSuccess)
+      return bail(fail(SDC_ERR_HIP, "hipFuncSetAttribute failed"));
+  if (hipFuncSetAttribute((const void*)k_coarse_inverse<true>,
                           hipFuncAttributeMaxDynamicSharedMemorySize, (int)kCoarseInvLds) !=
           hipSuccess)
     return bail(fail(SDC_ERR_HIP, "hipFuncSetAttribute failed"));
@@ -1624,6 +1842,7 @@ int sdc_destroy(sdc_handle h) {
   dfree(h->ainv64); dfree(h->ainv32); dfree(h->gj_a); dfree(h->gj_f);
   dfree(h->tcx); dfree(h->tcy); dfree(h->tcz); dfree(h->tbd); dfree(h->trd); dfree(h->tidg);
   dfree(h->jpart);
+  dfree(h->tail_img); dfree(h->tail_tab);
   dfree(h->cset_dev);
   h->w32.release();
   h->w64.release();
@@ -1781,6 +2000,7 @@ int build_levels(sdc_handle_s* h, hipStream_t st, int nset) {
                        h->ainv64, h->ainv32, h->gj_f, h->astride);
   HIPCK(hipGetLastError());
   h->nset = nset;
+  h->tail_stale = true;
   h->sigma_set = true;
   h->mixed_stalled = false;
   return SDC_OK;
@@ -1826,6 +2046,7 @@ int sdc_vcycle(sdc_handle h, int dtype, const void* b, void* z, int ncol, void* 
   } else if (dtype == SDC_F32) {
     h->vstore = h->prm.vcycle_bf16;
     CK(ensure_work<float>(h, ncol));
+    CK(ensure_tail(h, st, h->vstore == 0));
     CK(vcycle0<float>(h, (const float*)b, (float*)z, ncol, false, nullptr, st));
   } else {
     return fail(SDC_ERR_ARG, "dtype must be SDC_F32 or SDC_F64");
@@ -1941,6 +2162,7 @@ int sdc_solve(sdc_handle h, const double* q, double* u, int ncol, const sdc_solv
   } else {
     h->vstore = h->prm.vcycle_bf16;
     CK(ensure_work<float>(h, ncol));
+    CK(ensure_tail(h, st));
     Work<float>& W = h->w32;
     hipLaunchKernelGGL(k_zero<double>, dim3(nblk(len)), blk, 0, st, u, len);
     hipLaunchKernelGGL(k_zero<unsigned>, dim3(nblk(l0.nN)), blk, 0, st, W.qmask, (size_t)l0.nN);
