@@ -639,18 +639,98 @@ __global__ __launch_bounds__(SDC_BLOCK) void k_restrict_axis(AxisXfer t, const i
       st_once(out + (size_t)(c0 + r) * ldo + n, (X)(wl * v[r][0] + v[r][1] + wh * v[r][2]));
 }
 
+// The y and z factors of the separable restriction in one pass: out = Pz^T Py^T in on the coarse
+// grid, in on the grid (coarse x, fine y, fine z); weights as in k_restrict_axis (tables of both
+// axes, OPD: wy over the input grid, wz over (coarse x, coarse y, fine z)).  What bounds it is
+// latency on all but the largest levels and cache bandwidth there; as two passes it cost one
+// more launch per level and visit (4-5 us) and a write and read of the intermediate (95 against
+// 69 us from 932,137 nodes x 128 columns).
+struct YzXfer {
+  uint32_t b0, a1, a2, b1, nout;  // coarse x; fine y, z; coarse y counts; coarse nodes
+  FastDiv f0, f1;                 // division by b0 and b1
+  int remap;
+  const int32_t* cset;  // operator sets: wy + cset[c] * wys, wz + cset[c] * wzs (null: one set)
+  uint32_t wys, wzs;
+};
+
+template <typename T, typename X, int R, bool OPD>
+__global__ __launch_bounds__(SDC_BLOCK) void k_restrict_yz(
+    YzXfer t, const int* __restrict__ riy, const int* __restrict__ riz,
+    const T* __restrict__ ly, const T* __restrict__ hy, const T* __restrict__ lz,
+    const T* __restrict__ hz, const T* __restrict__ wy, const T* __restrict__ wz,
+    const X* __restrict__ in, X* __restrict__ out, size_t ldi, size_t ldo, int ncol,
+    const int* __restrict__ done) {
+  if (done && ld_flag(done)) return;
+  SDC_NODE_PROLOGUE_R(t.nout, t.remap)
+  if (!live) return;
+  const uint32_t q = fdiv(n, t.f0);
+  const uint32_t I = n - q * t.b0;
+  const uint32_t K = fdiv(q, t.f1);
+  const uint32_t J = q - K * t.b1;
+  const uint32_t fj = (uint32_t)riy[J], fk = (uint32_t)riz[K];
+  const uint32_t yj[3] = {fj > 0 ? fj - 1 : 0, fj, fj + 1 < t.a1 ? fj + 1 : fj};
+  const uint32_t zk[3] = {fk > 0 ? fk - 1 : 0, fk, fk + 1 < t.a2 ? fk + 1 : fk};
+  if (OPD && t.cset) {
+    const size_t k = (size_t)t.cset[c0];
+    wy += k * t.wys;
+    wz += k * t.wzs;
+  }
+  uint32_t at[9];
+#pragma unroll
+  for (int c = 0; c < 3; ++c)
+#pragma unroll
+    for (int b = 0; b < 3; ++b) at[3 * c + b] = I + t.b0 * (yj[b] + t.a1 * zk[c]);
+  T wl[3], wh[3], zl = lz[K], zh = hz[K];
+  wl[0] = ly[J];
+  wh[0] = hy[J];
+  if (OPD) {
+    const T ml = (T)(wl[0] != T(0)), mh = (T)(wh[0] != T(0));
+    const uint32_t pz = I + t.b0 * J, pl = t.b0 * t.b1;
+    zl = wz[pz + pl * zk[0]] * (T)(zl != T(0));
+    zh = (T(1) - wz[pz + pl * zk[2]]) * (T)(zh != T(0));
+#pragma unroll
+    for (int c = 0; c < 3; ++c) {
+      wl[c] = wy[at[3 * c]] * ml;
+      wh[c] = (T(1) - wy[at[3 * c + 2]]) * mh;
+    }
+  } else {
+    wl[1] = wl[2] = wl[0];
+    wh[1] = wh[2] = wh[0];
+  }
+  T v[R][9];
+#pragma unroll
+  for (int r = 0; r < R; ++r) {
+    const X* col = col_ptr(in, ldi, c0, r, ncol);
+#pragma unroll
+    for (int m = 0; m < 9; ++m) v[r][m] = (T)col[at[m]];
+  }
+#pragma unroll
+  for (int r = 0; r < R; ++r)
+    if (c0 + r < ncol) {
+      T y[3];
+#pragma unroll
+      for (int c = 0; c < 3; ++c) y[c] = wl[c] * v[r][3 * c] + v[r][3 * c + 1] + wh[c] * v[r][3 * c + 2];
+      st_once(out + (size_t)(c0 + r) * ldo + n, (X)(zl * y[0] + y[1] + zh * y[2]));
+    }
+}
+
 // xf += P xc, one work-item per coarse node (I, J, K): it updates the fine nodes it owns, the
 // fine nodes from its own fine position up to (not including) the next coarse node's along
 // every axis (1 or 2 per axis, up to 8), all of which interpolate from the 2x2x2 coarse nodes
-// (I..I+1, J..J+1, K..K+1): one coarse load per owned fine node and column, and the weight
-// loads are shared by the owned nodes and the R columns.  A fine node's value is
-//   xf + sum over the parent-cell corners m = a + 2b + 4c (in that order) of w_m xc_m,
-//   w_m = (a ? fx : 1 - fx) (b ? fy_a : 1 - fy_a) (c ? fz_ab : 1 - fz_ab)
-// with fx the weight of the right x parent at the fine node, fy_a the weight of the upper y
-// parent on the Py grid at x parent a, fz_ab that of the upper z parent on the Pz grid
-// (operator-dependent: t.wx, t.wy, t.wz; else the geometric tables pwx, pwy, pwz).  An owned
-// node coincident with the coarse grid along an axis has weight 0 on the next coarse node
-// there, whose index is clamped into the grid.
+// (I..I+1, J..J+1, K..K+1), along z, then y, then x, each step with the weight of the upper
+// parent: fz of the four (x, y) parents on the Pz grid, fy of the two x parents on the Py grid,
+// fx at the fine node (operator-dependent: t.wz, t.wy, t.wx; else the geometric tables).  Where
+// the coarse cell spans one fine cell along an axis the second node is the first again (and so
+// are the coarse parents, whose weights then do not matter) and is not written.
+// Every load goes out before the first store: with the eight fine nodes updated one after the
+// other, each load waited for the store before it (they may alias), eight memory round trips on
+// levels too small to hide them (12-15 us per launch where the other kernels take 5; on 932,137
+// nodes x 128 columns 238 us against 165 now).  The two
+// nodes of an x pair are read and written together (a pair may start at an odd element).
+template <typename X>
+struct XPair {
+  X a, b;
+};
 template <typename T, typename X, int R, bool OPD>
 __global__ __launch_bounds__(SDC_BLOCK) void k_prolong_own(Xfer<T> ta, const X* __restrict__ xc,
                                                            X* __restrict__ xf, size_t ldf,
@@ -665,82 +745,79 @@ __global__ __launch_bounds__(SDC_BLOCK) void k_prolong_own(Xfer<T> ta, const X* 
   const uint32_t K = fdiv(rr, t.cfy);
   const uint32_t J = rr - K * t.cn1y;
   const bool hx = I + 1 < t.cn1x, hy = J + 1 < t.cn1y, hz = (K + 1) * t.cplane < t.cN;
-  const uint32_t Ip = hx ? I + 1 : I, Jp = hy ? J + 1 : J, Kp = hz ? K + 1 : K;
   const uint32_t i0 = (uint32_t)t.rix[I], j0 = (uint32_t)t.riy[J], k0 = (uint32_t)t.riz[K];
   // owned nodes per axis: 2 where the coarse cell spans 2 fine cells
-  const bool ox = hx && (uint32_t)t.rix[Ip] == i0 + 2, oy = hy && (uint32_t)t.riy[Jp] == j0 + 2,
-             oz = hz && (uint32_t)t.riz[Kp] == k0 + 2;
-  const uint32_t c000 = I + J * t.cn1x + K * t.cplane;
-  const uint32_t dx = Ip - I, dy = (Jp - J) * t.cn1x, dz = (Kp - K) * t.cplane;
+  const bool ox = hx && (uint32_t)t.rix[hx ? I + 1 : I] == i0 + 2,
+             oy = hy && (uint32_t)t.riy[hy ? J + 1 : J] == j0 + 2,
+             oz = hz && (uint32_t)t.riz[hz ? K + 1 : K] == k0 + 2;
+  const uint32_t dx = ox ? 1u : 0u, dy = oy ? t.cn1x : 0u, dz = oz ? t.cplane : 0u;
+  // fine rows (y, z offset b + 2 c) and the pair's first element: one before the node where it
+  // owns no second one, so that the pair stays inside the column
+  uint32_t row[4];
+#pragma unroll
+  for (int m = 0; m < 4; ++m)
+    row[m] = i0 + t.fn1x * (j0 + ((m & 1) && oy ? 1u : 0u) +
+                            t.fn1y * (k0 + (m >= 2 && oz ? 1u : 0u)));
+  const uint32_t back = !ox && row[0] > 0 ? 1u : 0u;
+  T fx[4], fy[2][2], fz[4];
+  if (OPD) {
+    const uint32_t py = I + t.cn1x * (j0 + (oy ? 1u : 0u) + t.fn1y * k0);
+    const uint32_t py1 = oz ? py + t.cn1x * t.fn1y : py;
+    const uint32_t pz = I + t.cn1x * J + t.cplane * (k0 + (oz ? 1u : 0u));
+#pragma unroll
+    for (int m = 0; m < 4; ++m) fx[m] = t.wx[row[m] + dx];
+    fy[0][0] = t.wy[py];
+    fy[0][1] = t.wy[py + dx];
+    fy[1][0] = t.wy[py1];
+    fy[1][1] = t.wy[py1 + dx];
+    fz[0] = t.wz[pz];
+    fz[1] = t.wz[pz + dx];
+    fz[2] = t.wz[pz + dy];
+    fz[3] = t.wz[pz + dy + dx];
+  } else {
+    fx[0] = fx[1] = fx[2] = fx[3] = t.pwx[i0 + dx];
+    fy[0][0] = fy[0][1] = fy[1][0] = fy[1][1] = t.pwy[j0 + (oy ? 1u : 0u)];
+    fz[0] = fz[1] = fz[2] = fz[3] = t.pwz[k0 + (oz ? 1u : 0u)];
+  }
   T cv[R][8];
+  XPair<X> fv[R][4];
 #pragma unroll
   for (int r = 0; r < R; ++r) {
-    const X* c = col_ptr(xc, ldc, c0, r, ncol);
-    cv[r][0] = (T)c[c000];
-    cv[r][1] = (T)c[c000 + dx];
-    cv[r][2] = (T)c[c000 + dy];
-    cv[r][3] = (T)c[c000 + dy + dx];
-    cv[r][4] = (T)c[c000 + dz];
-    cv[r][5] = (T)c[c000 + dz + dx];
-    cv[r][6] = (T)c[c000 + dz + dy];
-    cv[r][7] = (T)c[c000 + dz + dy + dx];
+    const X* c = col_ptr(xc, ldc, c0, r, ncol) + n;
+    cv[r][0] = (T)c[0];
+    cv[r][1] = (T)c[dx];
+    cv[r][2] = (T)c[dy];
+    cv[r][3] = (T)c[dy + dx];
+    cv[r][4] = (T)c[dz];
+    cv[r][5] = (T)c[dz + dx];
+    cv[r][6] = (T)c[dz + dy];
+    cv[r][7] = (T)c[dz + dy + dx];
+    const X* f = col_ptr((const X*)xf, ldf, c0, r, ncol);
+#pragma unroll
+    for (int m = 0; m < 4; ++m) __builtin_memcpy(&fv[r][m], f + (row[m] - back), sizeof(XPair<X>));
   }
 #pragma unroll
-  for (int cz = 0; cz < 2; ++cz) {
-    if (cz && !oz) break;
-    const uint32_t k = k0 + cz;
+  for (int r = 0; r < R; ++r) {
+    if (c0 + r >= ncol) break;
+    X* f = xf + (size_t)(c0 + r) * ldf;
+    const T* v = cv[r];
+    T z[4];
 #pragma unroll
-    for (int by = 0; by < 2; ++by) {
-      if (by && !oy) continue;
-      const uint32_t j = j0 + by;
-      // y weights of the two x parents at fine (j, k); z weights of the four (x, y) parents
-      T fy[2] = {T(0), T(0)}, fz[2][2] = {{T(0), T(0)}, {T(0), T(0)}};
-      if (by) {
-        if (OPD) {
-          const uint32_t py = I + t.cn1x * (j + t.fn1y * k);
-          fy[0] = t.wy[py];
-          fy[1] = t.wy[py + dx];
-        } else {
-          fy[0] = fy[1] = t.pwy[j];
-        }
-      }
-      if (cz) {
-        if (OPD) {
-          const uint32_t pz = I + t.cn1x * J + t.cplane * k;
-          fz[0][0] = t.wz[pz];
-          fz[1][0] = t.wz[pz + dx];
-          fz[0][1] = t.wz[pz + dy];
-          fz[1][1] = t.wz[pz + dy + dx];
-        } else {
-          fz[0][0] = fz[1][0] = fz[0][1] = fz[1][1] = t.pwz[k];
-        }
-      }
+    for (int m = 0; m < 4; ++m) z[m] = v[m] + fz[m] * (v[m + 4] - v[m]);
 #pragma unroll
-      for (int ax = 0; ax < 2; ++ax) {
-        if (ax && !ox) continue;
-        const uint32_t f = i0 + ax + t.fn1x * (j + t.fn1y * k);
-        const T fx = ax ? (OPD ? t.wx[f] : t.pwx[i0 + 1]) : T(0);
-        T fv[R];
-#pragma unroll
-        for (int r = 0; r < R; ++r) fv[r] = (T)col_ptr((const X*)xf, ldf, c0, r, ncol)[f];
-        T w[8];
-#pragma unroll
-        for (int c = 0; c < 2; ++c)
-#pragma unroll
-          for (int b = 0; b < 2; ++b)
-#pragma unroll
-            for (int a = 0; a < 2; ++a)
-              w[a + 2 * b + 4 * c] = (a ? fx : T(1) - fx) * (b ? fy[a] : T(1) - fy[a]) *
-                                     (c ? fz[a][b] : T(1) - fz[a][b]);
-#pragma unroll
-        for (int r = 0; r < R; ++r) {
-          if (c0 + r < ncol) {
-            T acc = fv[r];
-#pragma unroll
-            for (int q = 0; q < 8; ++q) acc += w[q] * cv[r][q];
-            xf[(size_t)(c0 + r) * ldf + f] = (X)acc;
-          }
-        }
+    for (int m = 0; m < 4; ++m) {
+      const int by = m & 1, cz = m >> 1;
+      if ((by && !oy) || (cz && !oz)) continue;
+      const T p0 = cz ? z[0] : v[0], p1 = cz ? z[1] : v[1], p2 = cz ? z[2] : v[2],
+              p3 = cz ? z[3] : v[3];
+      const T q0 = by ? p0 + fy[cz][0] * (p2 - p0) : p0;
+      const T q1 = by ? p1 + fy[cz][1] * (p3 - p1) : p1;
+      const X a = back ? fv[r][m].b : fv[r][m].a;
+      if (ox) {
+        const XPair<X> o{(X)((T)a + q0), (X)((T)fv[r][m].b + q0 + fx[m] * (q1 - q0))};
+        __builtin_memcpy(f + row[m], &o, sizeof o);
+      } else {
+        f[row[m]] = (X)((T)a + q0);
       }
     }
   }

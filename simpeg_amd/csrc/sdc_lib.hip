@@ -896,22 +896,32 @@ int ensure_tail(sdc_handle_s* h, hipStream_t st, bool at0 = true) {
   return SDC_OK;
 }
 
-// Columns per work-item of the stencil kernels: automatic = 4 (measured on MI355X: the
-// smoothing steps run 4 % faster than with 8, the Krylov step the same; 2 is slower).
-int pick_r(const sdc_handle_s* h, int ncol) {
-  int r = h->prm.rhs_per_thread;
-  if (r == 1 || r == 2 || r == 4 || r == 8) return r;
-  if (ncol >= 4) return 4;
-  if (ncol >= 2) return 2;
-  return 1;
+// Fewer columns per work-item where a launch over nN nodes would have less than two work-groups
+// per CU: what a column group saves in coefficient loads does not matter there, the chip is idle
+// (fp64, 32 columns on 54,675 nodes: 3,630 us per solve with 4 columns everywhere, 3,465 by this
+// rule).
+int fill_chip(uint32_t nN, int ncol, int r) {
+  constexpr size_t kGroups = 512;
+  while (r > 1 && (size_t)nblk(nN) * (size_t)((ncol + r - 1) / r) < kGroups) r >>= 1;
+  return r;
 }
 
-// columns per work-item of the grid-transfer kernels: automatic = 8 (their gathers share one
-// index computation across the columns; 4 makes the restriction 15 % slower)
-int pick_rx(const sdc_handle_s* h, int ncol) {
+// Columns per work-item of the stencil kernels over nN nodes: automatic = 4 (measured on MI355X:
+// the smoothing steps run 4 % faster than with 8, the Krylov step the same; 2 is slower), fewer on
+// small levels.
+int pick_r(const sdc_handle_s* h, int ncol, uint32_t nN) {
+  int r = h->prm.rhs_per_thread;
+  if (r == 1 || r == 2 || r == 4 || r == 8) return r;
+  return fill_chip(nN, ncol, ncol >= 3 ? 4 : ncol);
+}
+
+// Columns per work-item of the grid-transfer kernels over nN coarse nodes: automatic = 8 (at
+// 932,137 nodes x 128 columns: prolongation 165 us, y and z restriction 69 us, against 180 and 75
+// with 4), fewer on small levels.
+int pick_rx(const sdc_handle_s* h, int ncol, uint32_t nN) {
   const int r = h->prm.xfer_rhs_per_thread;
   if (r == 1 || r == 2 || r == 4 || r == 8) return r;
-  return ncol >= 8 ? 8 : pick_r(h, ncol);
+  return fill_chip(nN, ncol, ncol >= 5 ? 8 : ncol >= 3 ? 4 : ncol);
 }
 
 // Stencil kernels of the fp32 solver: R columns per work-item, or (col_loop 8 / 16) a loop over
@@ -1011,7 +1021,7 @@ template <typename T, typename S, typename B, typename O>
 int vcycle(sdc_handle_s* h, int l, const B* b, O* x, int ncol, bool dot_out, const int* done,
            hipStream_t st) {
   Work<T>& W = work_of<T>(h);
-  const int R = pick_r(h, ncol);
+  const int R = pick_r(h, ncol, h->L[l].nN);
   const int G_ = pick_g(h, ncol);
   const Level& lv = h->L[l];
   const int nl = (int)h->L.size();
@@ -1096,7 +1106,7 @@ int vcycle(sdc_handle_s* h, int l, const B* b, O* x, int ncol, bool dot_out, con
   const Level& cl = h->L[l + 1];
   S* const cb = (S*)W.b[l + 1];
   S* const cx = (S*)W.xs[l + 1];
-  const int RX = pick_rx(h, ncol);
+  const int RX = pick_rx(h, ncol, cl.nN);
   auto post_smooth = [&](bool fin) {
     const int nsteps = fin ? nu2 : num;
     for (int k = 0; k < nsteps; ++k) {
@@ -1160,6 +1170,33 @@ int vcycle(sdc_handle_s* h, int l, const B* b, O* x, int ncol, bool dot_out, con
       const S* src = res;
       for (int p = 0; p < na; ++p) {
         const int a = axes[p];
+        if (a == 1 && p + 2 == na) {
+          // y and z together (the last two axes)
+          YzXfer yz{};
+          yz.b0 = dims[0]; yz.a1 = dims[1]; yz.a2 = dims[2];
+          yz.b1 = cdims[1];
+          yz.nout = cl.nN;
+          yz.f0 = make_fastdiv(yz.b0);
+          yz.f1 = make_fastdiv(yz.b1);
+          yz.remap = h->prm.xcd_remap != 0;
+          yz.cset = h->cur_cset;
+          yz.wys = t.wys;
+          yz.wzs = t.wzs;
+          prof_begin(h, rtag, st);
+#define SDC_RESTRICT_YZ(OPD)                                                                     \
+  DISPATCH_R(RX, launch(h, (k_restrict_yz<T, S, R, OPD>), grid2(cl.nN, ncol, RX), blk, 0, st, yz, \
+                        t.riy, t.riz, t.rly, t.rhy, t.rlz, t.rhz, t.wy, t.wz, src, cb, lv.ld,     \
+                        cl.ld, ncol, done))
+          if (t.wx) {
+            SDC_RESTRICT_YZ(true);
+          } else {
+            SDC_RESTRICT_YZ(false);
+          }
+#undef SDC_RESTRICT_YZ
+          prof_end(h, rtag, st,
+                   ((double)yz.b0 * yz.a1 * yz.a2 + (double)cl.nN) * cols * sS);
+          break;
+        }
         const bool lastp = p == na - 1;
         S* dst = lastp ? cb : (src == res ? oth : res);
         AxisXfer ax{};
@@ -1298,7 +1335,7 @@ int pcg(sdc_handle_s* h, T* x, int ncol, double tol, int maxit, const int* col_m
         hipStream_t st) {
   Work<T>& W = work_of<T>(h);
   const Level& l0 = h->L[0];
-  const int R = pick_r(h, ncol);
+  const int R = pick_r(h, ncol, h->L[0].nN);
   const int G_ = pick_g(h, ncol);
   const dim3 g = grid2(l0.nN, ncol, R);
   const dim3 blk(SDC_BLOCK);
@@ -1392,7 +1429,7 @@ int pcg_reliable(sdc_handle_s* h, const double* q, double* u, int ncol, const sd
   CK(ensure_tail(h, st));
   Work<float>& W = h->w32;
   const Level& l0 = h->L[0];
-  const int R = pick_r(h, ncol);
+  const int R = pick_r(h, ncol, h->L[0].nN);
   const int G_ = pick_g(h, ncol);
   const dim3 g = grid2(l0.nN, ncol, R);
   const dim3 blk(SDC_BLOCK);
@@ -2016,7 +2053,7 @@ int sdc_apply(sdc_handle h, int dtype, const void* x, void* y, int ncol, void* s
   DeviceGuard dg(h->device);
   hipStream_t st = (hipStream_t)stream;
   const Level& l0 = h->L[0];
-  const int R = pick_r(h, ncol);
+  const int R = pick_r(h, ncol, h->L[0].nN);
   const dim3 g = grid2(l0.nN, ncol, R);
   if (dtype == SDC_F64) {
     const Sten<double> s = make_sten<double>(h, 0, 2);
@@ -2069,7 +2106,7 @@ int sdc_solve(sdc_handle h, const double* q, double* u, int ncol, const sdc_solv
   DeviceGuard dg(h->device);
   hipStream_t st = (hipStream_t)stream;
   const Level& l0 = h->L[0];
-  const int R = pick_r(h, ncol);
+  const int R = pick_r(h, ncol, h->L[0].nN);
   const dim3 g = grid2(l0.nN, ncol, R);
   const dim3 blk(SDC_BLOCK);
   const uint32_t nbx = nblk(l0.nN);
@@ -2266,7 +2303,7 @@ int sdc_jvec_rhs(sdc_handle h, const double* dsig, const double* u, double* out,
   s.fx = make_fastdiv(l0.n1x); s.fy = make_fastdiv(l0.n1y);
   s.pin0 = 0;
   s.remap = h->prm.xcd_remap != 0;
-  const int R = pick_r(h, ncol);
+  const int R = pick_r(h, ncol, h->L[0].nN);
   DISPATCH_R(R, hipLaunchKernelGGL((k_apply<double, R, false>), grid2(l0.nN, ncol, R),
                                    dim3(SDC_BLOCK), 0, st, s, u, out, l0.ld, ncol,
                                    (double*)nullptr, (const int*)nullptr));
