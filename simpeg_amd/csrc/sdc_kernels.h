@@ -79,7 +79,16 @@ __device__ __forceinline__ bool set_changes(const Sten<T>& sa, int c, int cprev)
 #define SDC_CTL_MAXIT 8
 #define SDC_CTL_WINDOW 9
 #define SDC_CTL_FOLD 10
+// host copy only: NOTE is the last note a solve left for the host, a sequence number that grows
+// within the solve above SDC_NOTE_BITS flag bits -- one word, so that one store is the message
+// and needs no fence (written while later kernels of the iteration still run)
+#define SDC_CTL_NOTE 11
 #define SDC_CTL_N 16
+#define SDC_NOTE_BITS 3
+#define SDC_NOTE_STOP 1  // the solve stops
+#define SDC_NOTE_UPD 1   // k_norm_decide: a reliable update is due
+#define SDC_NOTE_FOLD 2  // k_norm_decide: a fold is due (full ring)
+#define SDC_NOTE_ANY 4   // k_norm_decide: some column is active
 // doubles after the ints: the largest true relative residual of the previous update and of the
 // last one, tol^2 and reliable_delta^2
 #define SDC_DCTL_MPREV 0
@@ -91,6 +100,11 @@ __device__ __forceinline__ bool set_changes(const Sten<T>& sa, int c, int cprev)
 __device__ __forceinline__ double* ctl_dbl(int* ctl) { return (double*)(ctl + SDC_CTL_N); }
 __device__ __forceinline__ const double* ctl_dbl(const int* ctl) {
   return (const double*)(ctl + SDC_CTL_N);
+}
+
+__device__ __forceinline__ void leave_note(int* hctl, int seq, int flags) {
+  __hip_atomic_store(hctl + SDC_CTL_NOTE, (seq << SDC_NOTE_BITS) | flags, __ATOMIC_RELAXED,
+                     __HIP_MEMORY_SCOPE_SYSTEM);
 }
 
 // a reliable update runs in this iteration
@@ -1211,7 +1225,8 @@ __device__ __forceinline__ void wave_sums(const double* __restrict__ p, uint32_t
 // when every active column's |r|^2 passed tol^2 |q|^2, some active column's dropped by
 // delta^2 since its last replacement (rmax), the iteration limit is reached, or `window`
 // iterations passed without an update.  Otherwise, when all nslot slots of the ring are
-// pending, it asks for a fold alone (the next iteration writes the oldest slot).
+// pending, it asks for a fold alone (the next iteration writes the oldest slot).  The decision
+// also goes to the host as a note (hctl: pinned memory, may be null), sequence number 2 it.
 __global__ __launch_bounds__(SDC_FIN_THREADS) void k_norm_decide(const double* __restrict__ partial,
                                                                  uint32_t nbx,
                                                                  double* __restrict__ rr,
@@ -1219,12 +1234,13 @@ __global__ __launch_bounds__(SDC_FIN_THREADS) void k_norm_decide(const double* _
                                                                  const double* __restrict__ qn2,
                                                                  const double* __restrict__ rmax,
                                                                  const int* __restrict__ active,
-                                                                 int ncol, int nslot) {
+                                                                 int ncol, int nslot,
+                                                                 int* __restrict__ hctl) {
   if (ld_flag(ctl + SDC_CTL_STOP)) return;
   const double tol2 = ld_flag(ctl_dbl(ctl) + SDC_DCTL_TOL2);
   const double delta2 = ld_flag(ctl_dbl(ctl) + SDC_DCTL_DELTA2);
   const int maxit = ld_flag(ctl + SDC_CTL_MAXIT), window = ld_flag(ctl + SDC_CTL_WINDOW);
-  int cand = 1, drop = 0;
+  int cand = 1, drop = 0, any = 0;
   constexpr int NW = SDC_FIN_THREADS / 64;
   for (int c0 = (int)threadIdx.x >> 6; c0 < ncol; c0 += SDC_FIN_COLS * NW) {
     double vs[SDC_FIN_COLS];
@@ -1236,12 +1252,14 @@ __global__ __launch_bounds__(SDC_FIN_THREADS) void k_norm_decide(const double* _
       const double v = vs[k];
       if ((threadIdx.x & 63) == 0) rr[c] = v;
       if (!active[c]) continue;
+      any = 1;
       if (v > tol2 * qn2[c]) cand = 0;
       if (v <= delta2 * rmax[c]) drop = 1;
     }
   }
   cand = __syncthreads_and(cand);
   drop = __syncthreads_or(drop);
+  if (hctl) any = __syncthreads_or(any);
   if (threadIdx.x == 0) {
     const int it = ld_flag(ctl + SDC_CTL_IT) + 1;
     ctl[SDC_CTL_IT] = it;
@@ -1249,8 +1267,12 @@ __global__ __launch_bounds__(SDC_FIN_THREADS) void k_norm_decide(const double* _
     ctl[SDC_CTL_PEND] = pend;
     const int upd =
         (cand || drop || it >= maxit || it - ld_flag(ctl + SDC_CTL_LAST) >= window) ? 1 : 0;
+    const int fold = (!upd && pend >= nslot) ? 1 : 0;
     ctl[SDC_CTL_UPD] = upd;
-    ctl[SDC_CTL_FOLD] = (!upd && pend >= nslot) ? 1 : 0;
+    ctl[SDC_CTL_FOLD] = fold;
+    if (hctl)
+      leave_note(hctl, 2 * it,
+                 upd * SDC_NOTE_UPD | fold * SDC_NOTE_FOLD | any * SDC_NOTE_ANY);
   }
 }
 
@@ -1260,7 +1282,7 @@ __global__ __launch_bounds__(SDC_FIN_THREADS) void k_norm_decide(const double* _
 // at the iteration limit, or when the largest true relative residual fell more slowly since the
 // previous update than 2^-SDC_STALL_RATE per iteration (the caller continues in fp64).  At the
 // stop the control block is also written to hctl (pinned host memory, may be null) for the host
-// to read.
+// to read, and every update leaves a note there (sequence number 2 it + 1).
 // The rate: an fp64 iteration costs 2.5-3 mixed ones and gains about 2.8 octaves of residual
 // (10 decades in 12 iterations), so a mixed phase below a quarter of that is slower than fp64.
 // Ordinary models gain 2.2 to 3.7 octaves per mixed iteration, a block of contrast 1e3 1.5, one
@@ -1348,7 +1370,7 @@ __global__ __launch_bounds__(SDC_FIN_THREADS) void k_true_after(const double* __
       if (hctl) {
         // the stop flag goes last, after a system-scope fence
         for (int i = 0; i < SDC_CTL_N; ++i)
-          if (i != SDC_CTL_STOP) hctl[i] = ld_flag(ctl + i);
+          if (i != SDC_CTL_STOP && i != SDC_CTL_NOTE) hctl[i] = ld_flag(ctl + i);
         double* hd = (double*)(hctl + SDC_CTL_N);
         for (int i = 0; i < SDC_DCTL_N; ++i) hd[i] = ld_flag(dctl + i);
         __threadfence_system();
@@ -1358,6 +1380,7 @@ __global__ __launch_bounds__(SDC_FIN_THREADS) void k_true_after(const double* __
       dctl[SDC_DCTL_MPREV] = m;
       ctl[SDC_CTL_LAST] = it;
     }
+    if (hctl) leave_note(hctl, 2 * it + 1, reason ? SDC_NOTE_STOP : 0);
   }
 }
 
@@ -1422,8 +1445,8 @@ __global__ __launch_bounds__(SDC_BLOCK) void k_fin_alpha(const double* __restric
 
 // convergence test |r| <= tol |b| per column (tol^2 from the control block ctl); the last
 // work-group counts the iteration (counters[4]) and publishes the number of still-active columns
-// and the stop flag: all converged, or counters[5] iterations done (device copy and host-mapped
-// copy)
+// and the stop flag: all converged, or counters[5] iterations done (also as a note to the host in
+// hctl, pinned memory, may be null)
 __global__ __launch_bounds__(SDC_BLOCK) void k_fin_rr(const double* __restrict__ partial,
                                                       uint32_t nbx,
                                                       const double* __restrict__ bnorm2,
@@ -1431,7 +1454,7 @@ __global__ __launch_bounds__(SDC_BLOCK) void k_fin_rr(const double* __restrict__
                                                       double* __restrict__ rr,
                                                       int* __restrict__ active,
                                                       int* __restrict__ counters, int* done,
-                                                      int* host_flag) {
+                                                      int* __restrict__ hctl) {
   if (ld_flag(done)) return;
   const double tol2 = ld_flag(ctl_dbl(ctl) + SDC_DCTL_TOL2);
   const int c = blockIdx.x;
@@ -1453,11 +1476,7 @@ __global__ __launch_bounds__(SDC_BLOCK) void k_fin_rr(const double* __restrict__
       counters[2] = nact;
       counters[0] = 0;
       counters[1] = 0;
-      if (host_flag) {
-        host_flag[0] = fin;
-        host_flag[1] = nact;
-        __threadfence_system();
-      }
+      if (hctl) leave_note(hctl, it, fin ? SDC_NOTE_STOP : 0);
     }
   }
 }

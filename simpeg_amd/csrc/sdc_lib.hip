@@ -20,6 +20,7 @@ constexpr int kRingSlots = 6;
 #include "simpeg_dc.h"
 
 #include <algorithm>
+#include <chrono>
 #include <cmath>
 #include <cstdio>
 #include <cstring>
@@ -1325,6 +1326,28 @@ int graph_run(sdc_handle_s* h, const void* b, void* x, int ncol, int variant, hi
   return SDC_OK;
 }
 
+// Wait until the solve's note to the host has reached sequence number `seq` and return it.  The
+// host reads the word itself for a while: a stream synchronisation returns some 10 us after the
+// kernel that wrote the note, as long as three kernels of a small problem take.  Past
+// kNoteSpin (large problems, where it does not matter) it gives the CPU back and synchronises.
+int wait_note(sdc_handle_s* h, hipStream_t st, int seq, int* note) {
+  constexpr auto kNoteSpin = std::chrono::microseconds(500);
+  const int* p = (const int*)h->h_ctl + SDC_CTL_NOTE;
+  auto there = [&] {
+    *note = __atomic_load_n(p, __ATOMIC_ACQUIRE);
+    return (*note >> SDC_NOTE_BITS) >= seq;
+  };
+  const auto t0 = std::chrono::steady_clock::now();
+  do {
+    for (int i = 0; i < 32; ++i) {
+      if (there()) return SDC_OK;
+      __builtin_ia32_pause();
+    }
+  } while (std::chrono::steady_clock::now() - t0 < kNoteSpin);
+  HIPCK(hipStreamSynchronize(st));
+  return there() ? SDC_OK : fail(SDC_ERR_STATE, "internal: the solve left no note");
+}
+
 // Preconditioned CG on ncol columns: rhs in W.r (overwritten by the residual), solution in x.
 // Each column stops when |r| <= tol |b|.  col_mask (device, may be null) excludes columns.
 // The convergence test and the iteration count live on the device (k_fin_rr), and every kernel
@@ -1343,6 +1366,10 @@ int pcg(sdc_handle_s* h, T* x, int ncol, double tol, int maxit, const int* col_m
   const size_t len = l0.ld * (size_t)ncol;
   int* done = W.counters + 3;
   const int K = std::max(1, (int)h->prm.check_every);
+  // One iteration at a time: the convergence test leaves the host a note, and the host launches
+  // the next iteration while the V-cycle behind the test still runs.
+  int* const hctl = K == 1 ? h->d_ctl : nullptr;
+  ((int*)h->h_ctl)[SDC_CTL_NOTE] = 0;
   // k_fin_rr sets the stop flag; the other kernels check it (a device-scope load at their start)
   // only when several iterations run between two host reads, since with one the kernels after
   // the test change nothing that the solve returns (x is final once r passed the test)
@@ -1381,8 +1408,7 @@ int pcg(sdc_handle_s* h, T* x, int ncol, double tol, int maxit, const int* col_m
            vdone);
     prof_end(h, SDC_PROF_UPDATE, s2, (double)l0.nN * ncol * 6 * sizeof(T));
     launch(h, k_fin_rr, dim3(ncol), blk, 0, s2, (const double*)W.partial, nblk4(l0.nN),
-           (const double*)W.bn2, (const int*)W.ctl, W.rr, W.active, W.counters, done,
-           (int*)nullptr);
+           (const double*)W.bn2, (const int*)W.ctl, W.rr, W.active, W.counters, done, hctl);
     CK(vcycle0<T>(h, W.r, W.z, ncol, true, vdone, s2));
     launch(h, k_fin_beta, dim3(ncol), blk, 0, s2, (const double*)W.partial, nbz, W.rz, W.beta,
            (const int*)W.active, 0, vdone);
@@ -1403,6 +1429,17 @@ int pcg(sdc_handle_s* h, T* x, int ncol, double tol, int maxit, const int* col_m
       CK(graph_run(h, W.counters, (void*)W.partial, ncol, variant, st, block));
     else
       CK(block(st));
+    if (hctl) {
+      int note = 0;
+      CK(wait_note(h, st, it + 1, &note));
+      if (iters) *iters = it + 1;
+      if (note & SDC_NOTE_STOP) {
+        HIPCK(hipGetLastError());
+        return SDC_OK;
+      }
+      if (it > maxit) return fail(SDC_ERR_STATE, "internal: PCG did not stop");
+      continue;
+    }
     HIPCK(hipMemcpyAsync(h->h_flag, W.counters + 3, 2 * sizeof(int), hipMemcpyDeviceToHost, st));
     HIPCK(hipStreamSynchronize(st));
     if (h->h_flag[0]) break;
@@ -1476,6 +1513,7 @@ int pcg_reliable(sdc_handle_s* h, const double* q, double* u, int ncol, const sd
   // the device writes the control block to h_ctl when it stops (d_ctl), and the host reads the
   // stop flag there after each block of iterations: cleared before the first launch
   ((int*)h->h_ctl)[SDC_CTL_STOP] = 0;
+  ((int*)h->h_ctl)[SDC_CTL_NOTE] = 0;
   // the right-hand-side node mask cleared and the control block set up in one launch; u is not
   // cleared: the first fold writes it (and its column padding) without reading it
   hipLaunchKernelGGL(k_mixed_init, dim3(nblk(l0.nN)), blk, 0, st, W.qmask, l0.nN, W.ctl, W.qu, q,
@@ -1489,23 +1527,35 @@ int pcg_reliable(sdc_handle_s* h, const double* q, double* u, int ncol, const sd
   // aux = |q|^2 and active = |q| > 0; rmax = |q|^2 (the residual at the last replacement)
   hipLaunchKernelGGL(k_fin_qnorm, dim3(ncol), blk, 0, st, (const double*)W.partial, nbx, W.aux,
                      W.rmax, W.active);
-  std::vector<double> h_qn(ncol);
-  HIPCK(hipMemcpyAsync(h_qn.data(), W.aux, ncol * sizeof(double), hipMemcpyDeviceToHost, st));
-  HIPCK(hipStreamSynchronize(st));
-  int nact = 0;
-  for (int c = 0; c < ncol; ++c) nact += h_qn[c] > 0.0;
   S.outer = 0;
   S.iters = 0;
   S.max_rel_res = 0.0;
-  S.converged = nact == 0;
-  if (nact == 0) {
+  S.converged = 0;
+  // no column has a right-hand side: u = 0
+  auto nothing = [&]() -> int {
     hipLaunchKernelGGL(k_zero<double>, dim3(nblk(len)), blk, 0, st, u, len);
+    S.converged = 1;
     return SDC_OK;
+  };
+  // One iteration between two host reads: the host waits for the decision's note and launches
+  // the fold, the fp64 residual and the stop test only when they are due (as launches that
+  // return at once they cost 11 us of an iteration's 60 at 2,550 nodes, 36 us at 932,137 nodes
+  // x 128 columns).  More iterations between reads (or one of the profiled classes that needs
+  // the decision, then one): the same kernels are always launched and test the control block.
+  const bool prof_upd = prof_on(h, SDC_PROF_REFINE) || prof_on(h, SDC_PROF_FOLD);
+  const int K = prof_upd ? 1 : std::max(1, (int)h->prm.check_every);
+  const bool notes = K == 1 && h->d_ctl;
+  if (!notes) {
+    std::vector<double> h_qn(ncol);
+    HIPCK(hipMemcpyAsync(h_qn.data(), W.aux, ncol * sizeof(double), hipMemcpyDeviceToHost, st));
+    HIPCK(hipStreamSynchronize(st));
+    int nact = 0;
+    for (int c = 0; c < ncol; ++c) nact += h_qn[c] > 0.0;
+    if (nact == 0) return nothing();
   }
   // storage 1, 4: the preconditioned residual z is bfloat16
   const bool zb = (vst == 1 || vst == 4) && h->L.size() > 1;
   __bf16* const z16 = (__bf16*)W.xb0;
-  const int K = std::max(1, (int)h->prm.check_every);
   // Early exits after the stop flag only matter when several iterations run between two host
   // reads of it (check_every > 1); the flag is read with a device-scope load at the start of
   // every kernel that checks it, which costs latency, so with one iteration per read the
@@ -1520,11 +1570,9 @@ int pcg_reliable(sdc_handle_s* h, const double* q, double* u, int ncol, const sd
                                                    : R;
   // Iteration: z = M r (z kept in the V-cycle storage type), beta, p = z + beta p and
   // q = A z + beta q in one pass (p into the next ring slot), alpha, r -= alpha q, the update
-  // decision, and the predicated fold of the pending directions into u (reliable update or
-  // full ring) and fp64 true residual (reliable update).
+  // decision; then (update) the fold of the pending directions into u (reliable update or
+  // full ring) and the fp64 true residual (reliable update).
   // Every launch goes through launch() so that the whole iteration can be recorded.
-  bool fold_fresh = true;  // profiled runs only: the next fold writes u without reading it
-  int fold_pend = 0;       // profiled runs only: directions the next fold reads
   const int S_ = W.nslot;
   const size_t slot_len = l0.ld * (size_t)W.ncap;
   // iteration `it` (0: the first) writes its search direction to ring slot it % S_
@@ -1579,27 +1627,20 @@ int pcg_reliable(sdc_handle_s* h, const double* q, double* u, int ncol, const sd
     prof_end(h, SDC_PROF_UPDATE, s, (double)l0.nN * ncol * (r16 ? 14 : 12));
     launch(h, k_norm_decide, dim3(1), dim3(SDC_FIN_THREADS), 0, s, (const double*)W.partial,
            gupd.x, W.rr, W.ctl, (const double*)W.aux, (const double*)W.rmax,
-           (const int*)W.active, ncol, S_);
-    // reliable update (every kernel below returns at once unless k_norm_decide asked for it).  A
-    // profiled run brackets the fold and the fp64 residual only when they do work, so it reads
-    // the decision on the host (graphs are off while profiling).
-    bool upd = true;
-    if (prof_on(h, SDC_PROF_REFINE) || prof_on(h, SDC_PROF_FOLD)) {
-      HIPCK(hipMemcpyAsync(h->h_ctl, W.ctlmem, SDC_CTL_N * sizeof(int), hipMemcpyDeviceToHost, s));
-      HIPCK(hipStreamSynchronize(s));
-      const int* hc = (const int*)h->h_ctl;
-      upd = hc[SDC_CTL_STOP] == 0 && hc[SDC_CTL_UPD] != 0;
-      fold_fresh = hc[SDC_CTL_UFRESH] != 0;
-      fold_pend = hc[SDC_CTL_PEND];
-    }
-    prof_begin(h, upd ? SDC_PROF_FOLD : -1, s);
+           (const int*)W.active, ncol, S_, notes ? h->d_ctl : nullptr);
+    return SDC_OK;
+  };
+  // Reliable update or fold (every kernel returns at once unless k_norm_decide asked for it);
+  // for profiled runs: fresh, u has not been written yet; pend, the directions folded
+  auto update = [&](hipStream_t s, int it, bool upd, bool fresh, int pend) -> int {
+    const int phi = it % S_;
+    prof_begin(h, SDC_PROF_FOLD, s);
     launch(h, k_ir_fold_ring,
            dim3((nblk4(l0.ld) + SDC_FOLD_CHUNKS - 1) / SDC_FOLD_CHUNKS, (uint32_t)ncol), blk, 0, s,
            (const double* const*)W.qu, (const float* const*)W.ptab, (const double*)W.ahist, S_,
            phi, (int)W.ncap, l0.ld, l0.nN, (const int*)W.ctl);
     // algorithmic bytes: the pending directions read, u read (unless fresh) and written
-    prof_end(h, upd ? SDC_PROF_FOLD : -1, s,
-             (double)l0.nN * ncol * (4.0 * fold_pend + (fold_fresh ? 8 : 16)));
+    prof_end(h, SDC_PROF_FOLD, s, (double)l0.nN * ncol * (4.0 * pend + (fresh ? 8 : 16)));
     prof_begin(h, upd ? SDC_PROF_REFINE : -1, s);
     // kIrChunks node blocks per work-group: most launches return at once (no update)
     DISPATCH_RG(R64, G_, launch(h, (k_ir_residual<float, R, false, G, kIrChunks>),
@@ -1614,31 +1655,60 @@ int pcg_reliable(sdc_handle_s* h, const double* q, double* u, int ncol, const sd
            nbx_ir, (const double*)W.aux, W.orr, W.rmax, W.active, W.ctl, ncol, h->d_ctl);
     return SDC_OK;
   };
-  // the first iteration (FIRST variants) is launched; later ones run check_every at a time,
-  // then the host reads the control block
-  CK(iteration(true, st, 0));
   // profiled kernel classes are bracketed by events, which cannot sit inside a graph
   const bool rec = h->prm.graph && h->prof_mask == 0;
   const int variant = 1000 + 16 * K + (zb ? 1 : 0) + (r16 ? 2 : 0) + 4 * (R64 == 8);
   const int* h_ctl = (const int*)h->h_ctl;
-  for (int done_it = 1;; done_it += K) {
-    auto block = [&](hipStream_t s) -> int {
-      for (int k = 0; k < K; ++k) CK(iteration(false, s, done_it + k));
-      return SDC_OK;
-    };
-    // a recorded block fixes its ring slots: one graph per starting slot
-    if (rec)
-      CK(graph_run(h, W.ctl, (void*)W.partial, ncol, variant + ((done_it % S_) << 16), st,
-                   block));
-    else
-      CK(block(st));
-    if (!h->d_ctl)
-      HIPCK(hipMemcpyAsync(h->h_ctl, W.ctlmem, (kCtlInts + SDC_DCTL_N) * sizeof(double),
-                           hipMemcpyDeviceToHost, st));
-    HIPCK(hipStreamSynchronize(st));
-    if (__atomic_load_n(h_ctl + SDC_CTL_STOP, __ATOMIC_ACQUIRE)) break;
-    // the device stops at maxit by itself; this bound only guards the host loop
-    if (done_it > maxit + K) return fail(SDC_ERR_STATE, "internal: mixed PCG did not stop");
+  // `first` iterations (the FIRST variants) are launched; later ones run K at a time, recorded (a
+  // recorded block fixes its ring slots: one graph per starting slot), then the host reads the
+  // decision
+  if (notes) {
+    int folded = 0;  // iterations whose directions are in u
+    for (int it = 0;; ++it) {
+      if (rec && it > 0)
+        CK(graph_run(h, W.ctl, (void*)W.partial, ncol, variant + ((it % S_) << 16), st,
+                     [&](hipStream_t s) -> int { return iteration(false, s, it); }));
+      else
+        CK(iteration(it == 0, st, it));
+      int note = 0;
+      CK(wait_note(h, st, 2 * (it + 1), &note));
+      if (it == 0 && !(note & SDC_NOTE_ANY)) return nothing();
+      if (note & (SDC_NOTE_UPD | SDC_NOTE_FOLD)) {
+        CK(update(st, it, note & SDC_NOTE_UPD, folded == 0, it + 1 - folded));
+        folded = it + 1;
+      }
+      if (note & SDC_NOTE_UPD) {
+        CK(wait_note(h, st, 2 * (it + 1) + 1, &note));
+        if (note & SDC_NOTE_STOP) break;
+      }
+      // the device stops at maxit by itself; this bound only guards the host loop
+      if (it > maxit) return fail(SDC_ERR_STATE, "internal: mixed PCG did not stop");
+    }
+    HIPCK(hipStreamSynchronize(st));  // the kernel that wrote the block has ended
+  } else {
+    CK(iteration(true, st, 0));
+    CK(update(st, 0, true, true, 1));
+    for (int done_it = 1;; done_it += K) {
+      auto block = [&](hipStream_t s) -> int {
+        for (int k = 0; k < K; ++k) {
+          CK(iteration(false, s, done_it + k));
+          CK(update(s, done_it + k, true, false, 1));
+        }
+        return SDC_OK;
+      };
+      if (rec)
+        CK(graph_run(h, W.ctl, (void*)W.partial, ncol, variant + ((done_it % S_) << 16), st,
+                     block));
+      else
+        CK(block(st));
+      if (!h->d_ctl)
+        HIPCK(hipMemcpyAsync(h->h_ctl, W.ctlmem, (kCtlInts + SDC_DCTL_N) * sizeof(double),
+                             hipMemcpyDeviceToHost, st));
+      HIPCK(hipStreamSynchronize(st));
+      if (__atomic_load_n(h_ctl + SDC_CTL_STOP, __ATOMIC_ACQUIRE)) break;
+      // the device stops at maxit by itself; this bound only guards the host loop
+      if (done_it > maxit + K) return fail(SDC_ERR_STATE, "internal: mixed PCG did not stop");
+    }
   }
   S.iters = std::min(h_ctl[SDC_CTL_IT], maxit);
   S.outer = h_ctl[SDC_CTL_OUTER];
