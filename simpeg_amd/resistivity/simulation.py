@@ -262,18 +262,23 @@ class Simulation3DNodal:
         self._sd_cache = (key, sd)
         return sd
 
-    def _sigma_deriv_T(self, g):
-        """sigmaDeriv^T g; a diagonal derivative (Exp, Identity, Reciprocal maps) as a product of
-        vectors instead of a transposed sparse product."""
+    def _sigma_deriv_diagonal(self):
+        """The diagonal of a diagonal sigmaDeriv (Exp, Identity, Reciprocal maps), else None."""
         sd = self.sigmaDeriv
         if self._sd_diag is None or self._sd_diag[0] is not sd:  # checked once per matrix
             n = sd.shape[0]
             diag = sd.shape[1] == n and sd.nnz == n and np.array_equal(
                 sd.indptr, np.arange(n + 1)) and np.array_equal(sd.indices, np.arange(n))
             self._sd_diag = (sd, diag)
-        if self._sd_diag[1]:
-            return sd.data * np.asarray(g, dtype=float).ravel()
-        return sd.T @ g
+        return sd.data if self._sd_diag[1] else None
+
+    def _sigma_deriv_T(self, g):
+        """sigmaDeriv^T g; a diagonal derivative as a product of vectors instead of a transposed
+        sparse product."""
+        d = self._sigma_deriv_diagonal()
+        if d is not None:
+            return d * np.asarray(g, dtype=float).ravel()
+        return self.sigmaDeriv.T @ g
 
     # ------------------------------------------------------------------ GPU state
     @property
@@ -514,6 +519,11 @@ class Simulation3DNodal:
             nD = pr["nD"]
             sd = self.sigmaDeriv
             J = np.empty((nD, sd.shape[1]))
+            # one parameter per cell: the rows are scaled on the GPU and copied to where they
+            # belong; through the sparse product they took 6 of 10 ms (90 data, 19,652 cells)
+            scale = self._sigma_deriv_diagonal()
+            if scale is not None:
+                scale = torch.as_tensor(-scale, dtype=torch.float64, device=eng.device)
             rows, nodes, w = pr["rows"], pr["nodes"], pr["w"]
             for c0 in range(0, nD, self.jchunk):
                 c1 = min(nD, c0 + self.jchunk)
@@ -524,7 +534,10 @@ class Simulation3DNodal:
                 rhs = eng.scatter(eng.scatter_csr(d, rp, sidx, sw), np.ones(k), k)
                 lam = self._solve(rhs, k)
                 G = eng.contract(f.u_block, lam, k, ucol=pr["data_src"][c0:c1], per_column=True)
-                J[c0:c1] = -(sd.T @ G.cpu().numpy().T).T
+                if scale is not None:
+                    torch.from_numpy(J[c0:c1]).copy_(G.mul_(scale))
+                else:
+                    J[c0:c1] = -(sd.T @ G.cpu().numpy().T).T
             self._Jmatrix = self._mini_data(J)
         return self._Jmatrix
 
