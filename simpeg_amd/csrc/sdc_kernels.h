@@ -443,13 +443,14 @@ __device__ __forceinline__ void restrict_weights(const Xfer<T>& t, uint32_t I, u
 // n: the point of the factor's grid; c: the fine level's conductances along AX (of one operator
 // set, as w64 and w32).  Run by k_coarsen_coef.
 template <int AX>
-__device__ __forceinline__ void interp_weight(const Xfer<double>& t, size_t n, uint32_t g0,
-                                              uint32_t g1, const double* __restrict__ c,
+__device__ __forceinline__ void interp_weight(const Xfer<double>& t, uint32_t n, FastDiv f0,
+                                              FastDiv f1, uint32_t g0, uint32_t g1,
+                                              const double* __restrict__ c,
                                               double* __restrict__ w64, float* __restrict__ w32) {
-  const uint32_t p0 = (uint32_t)(n % g0);
-  const size_t q = n / g0;
-  const uint32_t p1 = (uint32_t)(q % g1);
-  const uint32_t p2 = (uint32_t)(q / g1);
+  const uint32_t q = fdiv(n, f0);
+  const uint32_t p0 = n - q * g0;
+  const uint32_t p2 = fdiv(q, f1);
+  const uint32_t p1 = q - p2 * g1;
   // fine indices of the grid point: coarse x on the Py and Pz grids, coarse y on the Pz grid
   const uint32_t fi = AX == 0 ? p0 : (uint32_t)t.rix[p0];
   const uint32_t fj = AX == 2 ? (uint32_t)t.riy[p1] : p1;
@@ -1840,7 +1841,8 @@ struct InterpGrids {
   double* w64[3];
   float* w32[3];
   size_t wstride[3];
-  uint32_t g0[3], g1[3], g2[3];
+  uint32_t g0[3], g1[3], n[3];  // x and y counts, points
+  FastDiv f0[3], f1[3];         // division by g0 and g1
 };
 
 // Coarse-level conductances from fine ones (blockIdx.y = 0): along the edge direction the (one
@@ -1862,15 +1864,18 @@ __global__ __launch_bounds__(SDC_BLOCK) void k_coarsen_coef(Xfer<double> t,
                                                             size_t cstride, InterpGrids iw) {
   if (blockIdx.y > 0) {
     const int ax = (int)blockIdx.y - 1;
-    const size_t m = (size_t)blockIdx.x * SDC_BLOCK + threadIdx.x;
-    if (m >= (size_t)iw.g0[ax] * iw.g1[ax] * iw.g2[ax]) return;
+    const uint32_t m = blockIdx.x * SDC_BLOCK + threadIdx.x;
+    if (m >= iw.n[ax]) return;
     const size_t zf = (size_t)blockIdx.z * fstride, zw = (size_t)blockIdx.z * iw.wstride[ax];
+    const double* const fc = (ax == 0 ? fcx : ax == 1 ? fcy : fcz) + zf;
+    double* const w64 = iw.w64[ax] + zw;
+    float* const w32 = iw.w32[ax] + zw;
     if (ax == 0)
-      interp_weight<0>(t, m, iw.g0[0], iw.g1[0], fcx + zf, iw.w64[0] + zw, iw.w32[0] + zw);
+      interp_weight<0>(t, m, iw.f0[0], iw.f1[0], iw.g0[0], iw.g1[0], fc, w64, w32);
     else if (ax == 1)
-      interp_weight<1>(t, m, iw.g0[1], iw.g1[1], fcy + zf, iw.w64[1] + zw, iw.w32[1] + zw);
+      interp_weight<1>(t, m, iw.f0[1], iw.f1[1], iw.g0[1], iw.g1[1], fc, w64, w32);
     else
-      interp_weight<2>(t, m, iw.g0[2], iw.g1[2], fcz + zf, iw.w64[2] + zw, iw.w32[2] + zw);
+      interp_weight<2>(t, m, iw.f0[2], iw.f1[2], iw.g0[2], iw.g1[2], fc, w64, w32);
     return;
   }
   const uint32_t n = blockIdx.x * SDC_BLOCK + threadIdx.x;
@@ -1893,86 +1898,89 @@ __global__ __launch_bounds__(SDC_BLOCK) void k_coarsen_coef(Xfer<double> t,
   const double wx[3] = {t.rlx[I], 1.0, t.rhx[I]};
   const double wy[3] = {t.rly[J], 1.0, t.rhy[J]};
   const double wz[3] = {t.rlz[K], 1.0, t.rhz[K]};
-  auto fidx = [&](int a, int b, int c) -> size_t {
-    return (size_t)a + (size_t)b * t.fn1x + (size_t)c * t.fplane;
+  // clamped indices: what a weight of 0 leaves out is loaded all the same and not added
+  const size_t xi[3] = {(size_t)max(fi - 1, 0), (size_t)fi,
+                        (size_t)min(fi + 1, (int)t.fn1x - 1)};
+  const size_t yj[3] = {(size_t)max(fj - 1, 0) * t.fn1x, (size_t)fj * t.fn1x,
+                        (size_t)min(fj + 1, (int)t.fn1y - 1) * t.fn1x};
+  const size_t zk[3] = {(size_t)max(fk - 1, 0) * t.fplane, (size_t)fk * t.fplane,
+                        (size_t)min(fk + 1, (int)(t.fN / t.fplane) - 1) * t.fplane};
+  // the edge from the fine node f to the next coarse node along the axis of stride d (two: both)
+  auto edge = [](const double* __restrict__ c, size_t f, size_t d, bool two) -> double {
+    const double c1 = c[f], c2 = c[f + (two ? d : 0)], s = c1 + c2;
+    return !two ? c1 : s > 0.0 ? c1 * c2 / s : 0.0;
   };
-  auto series = [](double c1, double c2) -> double {
-    const double s = c1 + c2;
-    return s > 0.0 ? c1 * c2 / s : 0.0;
-  };
-  // x edges
-  double sx = 0.0;
-  if (I + 1 < t.cn1x) {
-    const int span = t.rix[I + 1] - fi;
-    for (int c = 0; c < 3; ++c) {
-      if (wz[c] == 0.0) continue;
-      for (int b = 0; b < 3; ++b) {
-        if (wy[b] == 0.0) continue;
-        const size_t f = fidx(fi, fj + b - 1, fk + c - 1);
-        const double e = (span == 2) ? series(fcx[f], fcx[f + 1]) : fcx[f];
-        sx += wy[b] * wz[c] * e;
-      }
+  const bool hx = I + 1 < t.cn1x, hy = J + 1 < t.cn1y, hz = K + 1 < cn1z;
+  const bool x2 = hx && t.rix[hx ? I + 1 : I] - fi == 2;
+  const bool y2 = hy && t.riy[hy ? J + 1 : J] - fj == 2;
+  const bool z2 = hz && t.riz[hz ? K + 1 : K] - fk == 2;
+  double sx = 0.0, sy = 0.0, sz = 0.0, sb = 0.0;
+#pragma unroll
+  for (int p = 0; p < 3; ++p)
+#pragma unroll
+    for (int q = 0; q < 3; ++q) {
+      const double ex = edge(fcx, xi[1] + yj[q] + zk[p], 1, x2);
+      const double ey = edge(fcy, xi[q] + yj[1] + zk[p], t.fn1x, y2);
+      const double ez = edge(fcz, xi[q] + yj[p] + zk[1], t.fplane, z2);
+      sx += hx && wy[q] * wz[p] != 0.0 ? wy[q] * wz[p] * ex : 0.0;
+      sy += hy && wx[q] * wz[p] != 0.0 ? wx[q] * wz[p] * ey : 0.0;
+      sz += hz && wx[q] * wy[p] != 0.0 ? wx[q] * wy[p] * ez : 0.0;
     }
-  }
-  double sy = 0.0;
-  if (J + 1 < t.cn1y) {
-    const int span = t.riy[J + 1] - fj;
-    for (int c = 0; c < 3; ++c) {
-      if (wz[c] == 0.0) continue;
+#pragma unroll
+  for (int c = 0; c < 3; ++c)
+#pragma unroll
+    for (int b = 0; b < 3; ++b)
+#pragma unroll
       for (int a = 0; a < 3; ++a) {
-        if (wx[a] == 0.0) continue;
-        const size_t f = fidx(fi + a - 1, fj, fk + c - 1);
-        const double e = (span == 2) ? series(fcy[f], fcy[f + t.fn1x]) : fcy[f];
-        sy += wx[a] * wz[c] * e;
+        const double w = wx[a] * wy[b] * wz[c], v = fbd[xi[a] + yj[b] + zk[c]];
+        sb += w != 0.0 ? w * v : 0.0;
       }
-    }
-  }
-  double sz = 0.0;
-  if (K + 1 < cn1z) {
-    const int span = t.riz[K + 1] - fk;
-    for (int b = 0; b < 3; ++b) {
-      if (wy[b] == 0.0) continue;
-      for (int a = 0; a < 3; ++a) {
-        if (wx[a] == 0.0) continue;
-        const size_t f = fidx(fi + a - 1, fj + b - 1, fk);
-        const double e = (span == 2) ? series(fcz[f], fcz[f + t.fplane]) : fcz[f];
-        sz += wx[a] * wy[b] * e;
-      }
-    }
-  }
-  double sb = 0.0;
-  for (int c = 0; c < 3; ++c) {
-    if (wz[c] == 0.0) continue;
-    for (int b = 0; b < 3; ++b) {
-      if (wy[b] == 0.0) continue;
-      for (int a = 0; a < 3; ++a) {
-        if (wx[a] == 0.0) continue;
-        sb += wx[a] * wy[b] * wz[c] * fbd[fidx(fi + a - 1, fj + b - 1, fk + c - 1)];
-      }
-    }
-  }
   ccx[n] = sx;
   ccy[n] = sy;
   ccz[n] = sz;
   cbd[n] = sb;
 }
 
-// Inverse of the coarsest level's operator, one work-group of 1024 per operator set (blockIdx.x:
-// coefficients + set * s.sstride, matrices + set * astride, scratch + set * nn):
-//   1. the dense operator a (row-major nn x nn; pin = 1: identity row / column 0), one row per
-//      work-item;
-//   2. in-place Gauss-Jordan elimination without pivoting (the operator is SPD), every pivot
-//      step updating all nn*nn entries of a and inv in parallel (f: the elimination factors);
-//   3. inv <- (inv + inv^T) / 2 into inv64 and its fp32 copy inv32.
-// SH: a, inv and f live in LDS ((2 nn^2 + nn) doubles of dynamic shared memory), so the pivot
-// steps do not go through L2; otherwise in the global scratch ga, gf and in inv64.
-template <bool SH>
-__global__ __launch_bounds__(1024) void k_coarse_inverse(Sten<double> s, double* __restrict__ ga,
+// Row n of the dense operator a (row-major nn x nn, cleared; pin = 1: identity row / column 0).
+__device__ __forceinline__ void coarse_row(const Sten<double>& s, uint32_t n,
+                                           double* __restrict__ a) {
+  double* row = a + (size_t)n * s.nN;
+  const NodeC<double> c = node_coef(s, n);
+  row[n] = c.d + ((c.wxm + c.wxp) + (c.wym + c.wyp) + (c.wzm + c.wzp));
+  if (c.ixm != n) row[c.ixm] = -c.wxm;
+  if (c.ixp != n) row[c.ixp] = -c.wxp;
+  if (c.iym != n) row[c.iym] = -c.wym;
+  if (c.iyp != n) row[c.iyp] = -c.wyp;
+  if (c.izm != n) row[c.izm] = -c.wzm;
+  if (c.izp != n) row[c.izp] = -c.wzp;
+}
+
+#define SDC_CINV_MAX 128  // nodes of k_coarse_inverse
+
+// v of lane `lane` (the same for the whole wavefront)
+__device__ __forceinline__ double lane_value(double v, int lane) {
+  const uint64_t b = __builtin_bit_cast(uint64_t, v);
+  const uint64_t lo = (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)b, lane);
+  const uint64_t hi = (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)(b >> 32), lane);
+  return __builtin_bit_cast(double, lo | (hi << 32));
+}
+
+// Inverse of the coarsest level's operator (up to 16 RB <= 64 CB nodes), one work-group of 1024
+// per operator set (blockIdx.x: coefficients + set * s.sstride, matrices + set * astride), into
+// inv64 and its fp32 copy inv32, made symmetric: in-place Gauss-Jordan elimination without
+// pivoting (the operator is SPD).  The nn pivot steps are a serial chain, so a step has one
+// barrier and little else: wavefront k holds the rows k + 16 i in registers, one or two columns
+// per lane, so the elimination factors of its rows are one lane's values; only the scaled pivot
+// row goes through LDS, in two halves.  (The same elimination on a matrix in LDS, with four
+// barriers a step and an integer division per entry, took 78 us for the coarsest level of a
+// 2,550-node mesh, now 19.)
+template <int RB, int CB>
+__global__ __launch_bounds__(1024) void k_coarse_inverse(Sten<double> s,
                                                          double* __restrict__ inv64,
                                                          float* __restrict__ inv32,
-                                                         double* __restrict__ gf,
                                                          size_t astride) {
   extern __shared__ __align__(16) double cinv_smem[];
+  __shared__ double prow[2][64 * CB];
   const size_t zo = (size_t)blockIdx.x * s.sstride;
   s.cx += zo;
   s.cy += zo;
@@ -1981,25 +1989,97 @@ __global__ __launch_bounds__(1024) void k_coarse_inverse(Sten<double> s, double*
   s.idg += zo;
   inv64 += (size_t)blockIdx.x * astride;
   inv32 += (size_t)blockIdx.x * astride;
-  const int N = (int)s.nN;
-  const int NN = N * N;
-  double* a = SH ? cinv_smem : ga + (size_t)blockIdx.x * astride;
-  double* inv = SH ? cinv_smem + NN : inv64;
-  double* f = SH ? cinv_smem + 2 * NN : gf + (size_t)blockIdx.x * N;
-  const int tid = threadIdx.x;
-  for (int n = tid; n < N; n += 1024) {
-    double* row = a + (size_t)n * N;
-    for (int m = 0; m < N; ++m) row[m] = 0.0;
-    const NodeC<double> c = node_coef(s, (uint32_t)n);
-    row[n] = c.d + ((c.wxm + c.wxp) + (c.wym + c.wyp) + (c.wzm + c.wzp));
-    if (c.ixm != (uint32_t)n) row[c.ixm] = -c.wxm;
-    if (c.ixp != (uint32_t)n) row[c.ixp] = -c.wxp;
-    if (c.iym != (uint32_t)n) row[c.iym] = -c.wym;
-    if (c.iyp != (uint32_t)n) row[c.iyp] = -c.wyp;
-    if (c.izm != (uint32_t)n) row[c.izm] = -c.wzm;
-    if (c.izp != (uint32_t)n) row[c.izp] = -c.wzp;
+  const int N = (int)s.nN, NN = N * N;
+  double* const a = cinv_smem;
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  for (int e = tid; e < NN; e += 1024) a[e] = 0.0;
+  __syncthreads();
+  if (tid < N) coarse_row(s, (uint32_t)tid, a);
+  __syncthreads();
+  double v[RB][CB];
+#pragma unroll
+  for (int i = 0; i < RB; ++i)
+#pragma unroll
+    for (int j = 0; j < CB; ++j) {
+      const int r = wave + 16 * i, c = lane + 64 * j;
+      v[i][j] = r < N && c < N ? a[r * N + c] : 0.0;
+    }
+#pragma unroll
+  for (int ip = 0; ip < RB; ++ip) {
+    for (int q = 0; q < 16; ++q) {
+      const int p = 16 * ip + q, jp = ip >> 2;  // the pivot's column p is lane p - 64 jp's
+      if (p >= N) break;
+      double* const row = prow[p & 1];
+      if (wave == q) {
+        const double inv = 1.0 / lane_value(v[ip][jp], p - 64 * jp);
+#pragma unroll
+        for (int j = 0; j < CB; ++j) {
+          const double w = lane + 64 * j == p ? inv : v[ip][j] * inv;
+          row[lane + 64 * j] = w;
+        }
+      }
+      __syncthreads();
+      double w[CB];
+#pragma unroll
+      for (int j = 0; j < CB; ++j) w[j] = row[lane + 64 * j];
+#pragma unroll
+      for (int i = 0; i < RB; ++i) {
+        const double f = lane_value(v[i][jp], p - 64 * jp);
+#pragma unroll
+        for (int j = 0; j < CB; ++j) {
+          const double old = lane + 64 * j == p ? 0.0 : v[i][j];
+          v[i][j] = i == ip && wave == q ? w[j] : old - f * w[j];
+        }
+      }
+    }
   }
-  for (int e = tid; e < NN; e += 1024) inv[e] = ((e / N) == (e % N)) ? 1.0 : 0.0;
+#pragma unroll
+  for (int i = 0; i < RB; ++i)
+#pragma unroll
+    for (int j = 0; j < CB; ++j) {
+      const int r = wave + 16 * i, c = lane + 64 * j;
+      if (r < N && c < N) a[r * N + c] = v[i][j];
+    }
+  __syncthreads();
+#pragma unroll
+  for (int i = 0; i < RB; ++i)
+#pragma unroll
+    for (int j = 0; j < CB; ++j) {
+      const int r = wave + 16 * i, c = lane + 64 * j;
+      if (r >= N || c >= N) continue;
+      const double m = 0.5 * (v[i][j] + a[c * N + r]);
+      inv64[r * N + c] = m;
+      inv32[r * N + c] = (float)m;
+    }
+}
+
+// The same for coarsest levels that have no room there, on global memory: the dense operator in
+// ga, its inverse built up in inv64, the elimination factors in gf (+ set * nn).
+__global__ __launch_bounds__(1024) void k_coarse_inverse_big(Sten<double> s,
+                                                             double* __restrict__ ga,
+                                                             double* __restrict__ inv64,
+                                                             float* __restrict__ inv32,
+                                                             double* __restrict__ gf,
+                                                             size_t astride) {
+  const size_t zo = (size_t)blockIdx.x * s.sstride;
+  s.cx += zo;
+  s.cy += zo;
+  s.cz += zo;
+  s.rd += zo;
+  s.idg += zo;
+  const int N = (int)s.nN, NN = N * N;
+  double* const a = ga + (size_t)blockIdx.x * astride;
+  double* const inv = inv64 + (size_t)blockIdx.x * astride;
+  float* const out32 = inv32 + (size_t)blockIdx.x * astride;
+  double* const f = gf + (size_t)blockIdx.x * N;
+  const int tid = threadIdx.x;
+  for (int e = tid; e < NN; e += 1024) {
+    a[e] = 0.0;
+    inv[e] = e / N == e % N ? 1.0 : 0.0;
+  }
+  __syncthreads();
+  for (int n = tid; n < N; n += 1024) coarse_row(s, (uint32_t)n, a);
   __syncthreads();
   for (int p = 0; p < N; ++p) {
     const double ip = 1.0 / a[p * N + p];
@@ -2027,10 +2107,10 @@ __global__ __launch_bounds__(1024) void k_coarse_inverse(Sten<double> s, double*
     const int r = e / N, c = e % N;
     if (c < r) continue;
     const double v = 0.5 * (inv[r * N + c] + inv[c * N + r]);
-    inv64[r * N + c] = v;
-    inv64[c * N + r] = v;
-    inv32[r * N + c] = (float)v;
-    inv32[c * N + r] = (float)v;
+    inv[r * N + c] = v;
+    inv[c * N + r] = v;
+    out32[r * N + c] = (float)v;
+    out32[c * N + r] = (float)v;
   }
 }
 

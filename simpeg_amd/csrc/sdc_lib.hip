@@ -152,10 +152,6 @@ struct Level {
 // doubles taken by the int part of a control block
 constexpr int kCtlInts = SDC_CTL_N * (int)sizeof(int) / (int)sizeof(double);
 
-// dynamic LDS of the coarsest inverse when it runs in LDS (160 KB: all a gfx950 work-group
-// may use)
-constexpr size_t kCoarseInvLds = 160 * 1024;
-
 template <typename T>
 struct Work {
   int ncap = 0;
@@ -1729,8 +1725,10 @@ int alloc_coarse_inverse(sdc_handle_s* h, int nset) {
   const size_t k = (size_t)nset, nc = (size_t)h->ncoarse;
   CK(dmalloc(&h->ainv64, h->astride * k));
   CK(dmalloc(&h->ainv32, h->astride * k));
-  CK(dmalloc(&h->gj_a, h->astride * k));
-  CK(dmalloc(&h->gj_f, nc * k));
+  if (nc > SDC_CINV_MAX) {
+    CK(dmalloc(&h->gj_a, h->astride * k));
+    CK(dmalloc(&h->gj_f, nc * k));
+  }
   return SDC_OK;
 }
 
@@ -1881,7 +1879,7 @@ int sdc_create(const sdc_mesh_desc* d, sdc_handle* out) {
   fill_level_dims(l0);
   h->L.push_back(l0);
   // coarsest level: at most 64 nodes by default (its dense inverse is rebuilt by one work-group
-  // at every sdc_set_sigma, O(n^3): 128 nodes took 240 us, 64 nodes ~40 us)
+  // at every sdc_set_sigma: 19 us for some 60 nodes)
   const uint32_t cmax = d->coarse_max > 0 ? (uint32_t)d->coarse_max : 64u;
   double hmin = 1e300;
   for (int a = 0; a < 3; ++a)
@@ -1929,8 +1927,8 @@ int sdc_create(const sdc_mesh_desc* d, sdc_handle* out) {
     h->d_ctl = nullptr;
     (void)hipGetLastError();
   }
-  // the fused coarse tail and the coarsest inverse may use all 160 KB of LDS (set once,
-  // outside any graph capture)
+  // LDS beyond the default limit for the fused coarse tail (all 160 KB) and the coarsest inverse
+  // (its matrix), set once, outside any graph capture
   const void* const big_lds[] = {
       (const void*)k_tail_cycle<float, float, 2>,   (const void*)k_tail_cycle<float, float, 4>,
       (const void*)k_tail_cycle<float, float, 8>,   (const void*)k_tail_cycle<float, __bf16, 2>,
@@ -1941,10 +1939,13 @@ int sdc_create(const sdc_mesh_desc* d, sdc_handle* out) {
     if (hipFuncSetAttribute(k, hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024) !=
         hipSuccess)
       return bail(fail(SDC_ERR_HIP, "hipFuncSetAttribute failed"));
-  if (hipFuncSetAttribute((const void*)k_coarse_inverse<true>,
-                          hipFuncAttributeMaxDynamicSharedMemorySize, (int)kCoarseInvLds) !=
-          hipSuccess)
-    return bail(fail(SDC_ERR_HIP, "hipFuncSetAttribute failed"));
+  const void* const cinv[] = {(const void*)k_coarse_inverse<2, 1>,
+                              (const void*)k_coarse_inverse<4, 1>,
+                              (const void*)k_coarse_inverse<8, 2>};
+  for (const void* k : cinv)
+    if (hipFuncSetAttribute(k, hipFuncAttributeMaxDynamicSharedMemorySize,
+                            SDC_CINV_MAX * SDC_CINV_MAX * (int)sizeof(double)) != hipSuccess)
+      return bail(fail(SDC_ERR_HIP, "hipFuncSetAttribute failed"));
   *out = h;
   return SDC_OK;
 }
@@ -2076,11 +2077,13 @@ int build_levels(sdc_handle_s* h, hipStream_t st, int nset) {
     for (int a = 0; a < 3; ++a) {
       iw.g0[a] = g[a][0];
       iw.g1[a] = g[a][1];
-      iw.g2[a] = g[a][2];
+      iw.n[a] = g[a][0] * g[a][1] * g[a][2];
+      iw.f0[a] = make_fastdiv(g[a][0]);
+      iw.f1[a] = make_fastdiv(g[a][1]);
       iw.w64[a] = w64[a];
       iw.w32[a] = w32[a];
       iw.wstride[a] = ws[a];
-      nb = std::max(nb, (size_t)nblk((size_t)g[a][0] * g[a][1] * g[a][2]));
+      nb = std::max(nb, (size_t)nblk(iw.n[a]));
     }
     hipLaunchKernelGGL(k_coarsen_coef, dim3((uint32_t)nb, 4, z), dim3(SDC_BLOCK), 0, st, t,
                        (const double*)f.cx64, (const double*)f.cy64, (const double*)f.cz64,
@@ -2107,14 +2110,19 @@ int build_levels(sdc_handle_s* h, hipStream_t st, int nset) {
   const Sten<double> sc = make_sten<double>(h, lc, 1);
   const size_t nc = h->ncoarse;
   if (sc.nN != nc) return fail(SDC_ERR_STATE, "internal: coarsest level size");
-  // the elimination in LDS when a, inv and the factors fit (nn <= 99 with 160 KB)
-  const size_t cinv_lds = (2 * nc * nc + nc) * sizeof(double);
-  if (cinv_lds <= kCoarseInvLds)
-    hipLaunchKernelGGL(k_coarse_inverse<true>, dim3(z), dim3(1024), cinv_lds, st, sc, h->gj_a,
-                       h->ainv64, h->ainv32, h->gj_f, h->astride);
+#define SDC_CINV(RB, CB)                                                                      \
+  hipLaunchKernelGGL((k_coarse_inverse<RB, CB>), dim3(z), dim3(1024), nc * nc * sizeof(double), st, sc, \
+                     h->ainv64, h->ainv32, h->astride)
+  if (nc > SDC_CINV_MAX)
+    hipLaunchKernelGGL(k_coarse_inverse_big, dim3(z), dim3(1024), 0, st, sc, h->gj_a, h->ainv64,
+                       h->ainv32, h->gj_f, h->astride);
+  else if (nc > 64)
+    SDC_CINV(8, 2);
+  else if (nc > 32)
+    SDC_CINV(4, 1);
   else
-    hipLaunchKernelGGL(k_coarse_inverse<false>, dim3(z), dim3(1024), 0, st, sc, h->gj_a,
-                       h->ainv64, h->ainv32, h->gj_f, h->astride);
+    SDC_CINV(2, 1);
+#undef SDC_CINV
   HIPCK(hipGetLastError());
   h->nset = nset;
   h->tail_stale = true;
