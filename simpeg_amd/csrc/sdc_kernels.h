@@ -938,6 +938,21 @@ __global__ __launch_bounds__(SDC_BLOCK) void k_update_xr4(T* const* xp, const T*
   if (threadIdx.x == 0) partial[(size_t)c * gridDim.x + blockIdx.x] = t;
 }
 
+// sum of nbx partials over the work-group
+__device__ __forceinline__ double block_sum(const double* __restrict__ part, uint32_t nbx) {
+  __shared__ double red[SDC_BLOCK / 64];
+  double v = 0.0;
+  for (uint32_t b = threadIdx.x; b < nbx; b += SDC_BLOCK) v += part[b];
+#pragma unroll
+  for (int off = 32; off > 0; off >>= 1) v += __shfl_down(v, off, 64);
+  if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = v;
+  __syncthreads();
+  double t = 0.0;
+#pragma unroll
+  for (int w = 0; w < SDC_BLOCK / 64; ++w) t += red[w];
+  return t;
+}
+
 // The mixed-precision PCG step that replaces "p = z + beta p; q = A p": by linearity
 // q = A z + beta q, so the stencil reads z (the preconditioner output, possibly bf16) instead of
 // p, and p, q are updated pointwise; partial sums of p.q per column.  The search directions
@@ -946,52 +961,98 @@ __global__ __launch_bounds__(SDC_BLOCK) void k_update_xr4(T* const* xp, const T*
 // into u (fp64) by k_ir_fold_ring, so no fp32 iterate is read and written every step.
 // FIRST: p = z, q = A z.  check_stop: return at once when ctl[STOP] is set (only needed when
 // several iterations run between host reads of the stop flag).
+// With in.part every work-group sums its columns' r.z partials itself (k_fin_beta otherwise),
+// while its stencil loads are under way; the first one of a column group also stores r.z.
+struct BetaIn {
+  const double* part;     // r.z partials, nb per column (null: beta holds the result)
+  uint32_t nb;
+  const double* rz_prev;  // r.z of the previous iteration
+  double* rz;             // r.z of this one
+  const int* active;
+};
+
 template <typename Z, int R, bool FIRST, int G = 1>
 __global__ __launch_bounds__(SDC_BLOCK) void k_apply_pq(Sten<float> sa, const Z* __restrict__ z,
                                                         const float* __restrict__ p_prev,
                                                         float* __restrict__ p_out,
                                                         float* __restrict__ q,
                                                         const double* __restrict__ beta,
-                                                        size_t ld, int ncol,
+                                                        BetaIn in, size_t ld, int ncol,
                                                         double* __restrict__ partial,
                                                         const int* __restrict__ ctl,
                                                         int check_stop) {
   if (check_stop && ld_flag(ctl + SDC_CTL_STOP)) return;
   SDC_NODE_PROLOGUE_C(sa.nN, sa.remap, R * G)
+  __shared__ double sbeta[R * G];
+  // wavefront w: the columns c0 + w, c0 + w + 4, ...
+  auto sum_beta = [&] {
+    const int lane = threadIdx.x & 63;
+    for (int k = (int)threadIdx.x >> 6; k < R * G; k += SDC_BLOCK / 64) {
+      const int c = min(c0 + k, ncol - 1);
+      double v = 0.0;
+      for (uint32_t b = lane; b < in.nb; b += 64) v += in.part[(size_t)c * in.nb + b];
+#pragma unroll
+      for (int off = 32; off > 0; off >>= 1) v += __shfl_xor(v, off, 64);
+      if (lane == 0) {
+        const double old = FIRST ? 0.0 : in.rz_prev[c];
+        sbeta[k] = !FIRST && in.active[c] && old != 0.0 ? v / old : 0.0;
+        if (bx == 0 && c0 + k < ncol) in.rz[c] = v;
+      }
+    }
+    __syncthreads();
+  };
+  auto beta_of = [&](int k) -> float { return (float)(in.part ? sbeta[k] : beta[c0 + k]); };
   double acc[R * G];
 #pragma unroll
   for (int r = 0; r < R * G; ++r) acc[r] = 0.0;
-  if (live) {
-    NodeC<float> c = node_coef(sten_col(sa, c0), n);
-#pragma unroll 2
-    for (int gq = 0; gq < G; ++gq) {
-      const int cg = c0 + gq * R;
-      if (cg >= ncol) break;
-      if (G > 1 && gq > 0 && set_changes(sa, cg, cg - R)) c = node_coef(sten_col(sa, cg), n);
-      float zc[R], az[R], po[R], qo[R];
+  NodeC<float> c;
+  float zc[R], az[R], po[R], qo[R];
+  auto load = [&](int cg) {
 #pragma unroll
-      for (int r = 0; r < R; ++r) {
-        if (!FIRST) {
-          const size_t o = (size_t)(cg + r < ncol ? cg + r : ncol - 1) * ld + n;
-          po[r] = ld_once(p_prev + o);
-          qo[r] = ld_once(q + o);
-        }
+    for (int r = 0; r < R; ++r) {
+      if (!FIRST) {
+        const size_t o = (size_t)(cg + r < ncol ? cg + r : ncol - 1) * ld + n;
+        po[r] = ld_once(p_prev + o);
+        qo[r] = ld_once(q + o);
       }
-      stencil_cols<float, R>(c, z, n, ld, cg, ncol, zc, az);
+    }
+    stencil_cols<float, R>(c, z, n, ld, cg, ncol, zc, az);
+  };
+  auto finish = [&](int cg, int k0) {
 #pragma unroll
-      for (int r = 0; r < R; ++r) {
-        if (cg + r < ncol) {
-          const size_t o = (size_t)(cg + r) * ld + n;
-          float pn = zc[r], qn = az[r];
-          if (!FIRST) {
-            const float be = (float)beta[cg + r];
-            pn += be * po[r];
-            qn += be * qo[r];
-          }
-          st_once(p_out + o, pn);
-          st_once(q + o, qn);
-          acc[gq * R + r] += (double)pn * (double)qn;
+    for (int r = 0; r < R; ++r) {
+      if (cg + r < ncol) {
+        const size_t o = (size_t)(cg + r) * ld + n;
+        float pn = zc[r], qn = az[r];
+        if (!FIRST) {
+          const float be = beta_of(k0 + r);
+          pn += be * po[r];
+          qn += be * qo[r];
         }
+        st_once(p_out + o, pn);
+        st_once(q + o, qn);
+        acc[k0 + r] += (double)pn * (double)qn;
+      }
+    }
+  };
+  if constexpr (G == 1) {
+    if (live) {
+      c = node_coef(sten_col(sa, c0), n);
+      load(c0);
+    }
+    if (in.part) sum_beta();
+    if (live) finish(c0, 0);
+  } else {
+    if (in.part) sum_beta();
+    if (live) {
+      c = node_coef(sten_col(sa, c0), n);
+#pragma unroll 2
+      for (int gq = 0; gq < G; ++gq) {
+        const int cg = c0 + gq * R;
+        if (cg >= ncol) break;
+        if (gq > 0 && set_changes(sa, cg, cg - R)) c = node_coef(sten_col(sa, cg), n);
+        load(cg);
+        finish(cg, gq * R);
       }
     }
   }
@@ -1001,19 +1062,27 @@ __global__ __launch_bounds__(SDC_BLOCK) void k_apply_pq(Sten<float> sa, const Z*
 // r -= alpha q and per-column |r|^2 partials: a work-group takes CH chunks of SDC_NODES4 nodes
 // (4 per work-item and chunk, all loads issued before the arithmetic), one partial per
 // work-group, so that the single-work-group decision sums few partials per column
-// (R16: also write a bfloat16 copy of r, the multigrid input)
+// (R16: also write a bfloat16 copy of r, the multigrid input).  With in.part every work-group
+// sums its column's p.q partials itself (k_fin_alpha otherwise); the first one stores alpha.
+struct AlphaIn {
+  const double* part;  // p.q partials, nb per column (null: alpha holds the result)
+  uint32_t nb;
+  const double* rz;
+  const int* active;
+  double* ahist;       // alpha out (the ring slot's)
+};
+
 template <bool R16, int CH>
 __global__ __launch_bounds__(SDC_BLOCK) void k_update_r4(float* __restrict__ r,
                                                          const float* __restrict__ q,
                                                          const double* __restrict__ alpha,
-                                                         size_t ld, uint32_t nN,
+                                                         AlphaIn in, size_t ld, uint32_t nN,
                                                          double* __restrict__ partial,
                                                          __bf16* __restrict__ r16,
                                                          const int* __restrict__ done) {
   if (done && ld_flag(done)) return;
   const int c = blockIdx.y;
   const size_t o = (size_t)c * ld;
-  const float al = (float)alpha[c];
   const uint32_t base = (blockIdx.x * CH * SDC_BLOCK + threadIdx.x) * 4;
   vec4_t<float> rv[CH], qv[CH];
 #pragma unroll
@@ -1024,6 +1093,15 @@ __global__ __launch_bounds__(SDC_BLOCK) void k_update_r4(float* __restrict__ r,
       qv[k] = *(const vec4_t<float>*)(q + o + n0);
     }
   }
+  double a;
+  if (in.part) {
+    const double pq = block_sum(in.part + (size_t)c * in.nb, in.nb);
+    a = in.active[c] && pq > 0.0 ? in.rz[c] / pq : 0.0;
+    if (blockIdx.x == 0 && threadIdx.x == 0) in.ahist[c] = a;
+  } else {
+    a = alpha[c];
+  }
+  const float al = (float)a;
   double acc = 0.0;
 #pragma unroll
   for (int k = 0; k < CH; ++k) {
@@ -1156,20 +1234,6 @@ __global__ __launch_bounds__(SDC_BLOCK) void k_zero(T* __restrict__ x, size_t le
 
 // ------------------------------------------------------------------------------------------
 // per-column scalar finalisation (one work-group per column, sums the block partials)
-
-__device__ __forceinline__ double block_sum(const double* __restrict__ part, uint32_t nbx) {
-  __shared__ double red[SDC_BLOCK / 64];
-  double v = 0.0;
-  for (uint32_t b = threadIdx.x; b < nbx; b += SDC_BLOCK) v += part[b];
-#pragma unroll
-  for (int off = 32; off > 0; off >>= 1) v += __shfl_down(v, off, 64);
-  if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = v;
-  __syncthreads();
-  double t = 0.0;
-#pragma unroll
-  for (int w = 0; w < SDC_BLOCK / 64; ++w) t += red[w];
-  return t;
-}
 
 // out[c] = sum of partials; mode 1 additionally initialises the PCG state
 __global__ __launch_bounds__(SDC_BLOCK) void k_fin_norm(const double* __restrict__ partial,

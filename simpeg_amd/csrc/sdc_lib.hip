@@ -152,6 +152,13 @@ struct Level {
 // doubles taken by the int part of a control block
 constexpr int kCtlInts = SDC_CTL_N * (int)sizeof(int) / (int)sizeof(double);
 
+// Mixed PCG on levels of up to this many 256-node blocks: the sums behind beta and alpha are taken
+// by every work-group that needs them instead of a launch of their own.  A launch costs 4.5-5 us;
+// so many partials are 8 KB of cached reads per work-group, which moves 24 KB of its own (2,550
+// nodes x 4 columns 687 us per solve with launches, 640 this way; a gradient on 22,050 nodes
+// 2,819 and 2,701; a Hessian product on 54,600, 214 blocks, 4,939 and 4,834).
+constexpr uint32_t kInlineSums = 256;
+
 template <typename T>
 struct Work {
   int ncap = 0;
@@ -191,11 +198,15 @@ struct Work {
   T* pr = nullptr;
   T** ptab = nullptr;
   double* ahist = nullptr;
+  // small problems: r.z of the ring's slots (nslot x ncap) and the p.q partials, apart from
+  // `partial` because work-groups still read the r.z partials there
+  double* rzh = nullptr;
+  double* pqpart = nullptr;
   int nslot = 0;
   void release() {
     dfree(x); dfree(r); dfree(z); dfree(p); dfree(q); dfree(r16);
     dfree(ctlmem); dfree(rmax); dfree(qu); dfree(xtab);
-    dfree(pr); dfree(ptab); dfree(ahist);
+    dfree(pr); dfree(ptab); dfree(ahist); dfree(rzh); dfree(pqpart);
     nslot = 0;
     ctl = nullptr;
     dctl = nullptr;
@@ -636,6 +647,10 @@ int ensure_work(sdc_handle_s* h, int ncol) {
     w.nslot = kRingSlots;
     CK(dmalloc(&w.pr, n0 * (size_t)w.nslot));
     CK(dmalloc(&w.ahist, (size_t)cap * w.nslot));
+    if (nb0 <= kInlineSums) {
+      CK(dmalloc(&w.rzh, (size_t)cap * w.nslot));
+      CK(dmalloc(&w.pqpart, nb0 * (size_t)cap));
+    }
     std::vector<T*> tab((size_t)w.nslot);
     for (int k = 0; k < w.nslot; ++k) tab[(size_t)k] = w.pr + (size_t)k * n0;
     CK(upload(&w.ptab, tab));
@@ -1569,6 +1584,7 @@ int pcg_reliable(sdc_handle_s* h, const double* q, double* u, int ncol, const sd
   // decision; then (update) the fold of the pending directions into u (reliable update or
   // full ring) and the fp64 true residual (reliable update).
   // Every launch goes through launch() so that the whole iteration can be recorded.
+  const bool inl = nbx <= kInlineSums;
   const int S_ = W.nslot;
   const size_t slot_len = l0.ld * (size_t)W.ncap;
   // iteration `it` (0: the first) writes its search direction to ring slot it % S_
@@ -1586,9 +1602,15 @@ int pcg_reliable(sdc_handle_s* h, const double* q, double* u, int ncol, const sd
     else
       rc = vcycle0<float>(h, W.r, W.z, ncol, true, stop, s);
     CK(rc);
-    launch(h, k_fin_beta, dim3(ncol), blk, 0, s, (const double*)W.partial, dot_blocks<float>(h),
-           W.rz, W.beta,
-           (const int*)W.active, first ? 1 : 0, stop);
+    BetaIn bin{};
+    double* const rz = inl ? W.rzh + (size_t)phi * W.ncap : W.rz;
+    double* const pqpart = inl ? W.pqpart : W.partial;
+    if (inl)
+      bin = BetaIn{W.partial, dot_blocks<float>(h),
+                   W.rzh + (size_t)((it + S_ - 1) % S_) * W.ncap, rz, W.active};
+    else
+      launch(h, k_fin_beta, dim3(ncol), blk, 0, s, (const double*)W.partial,
+             dot_blocks<float>(h), W.rz, W.beta, (const int*)W.active, first ? 1 : 0, stop);
     // the class covers the steady-state launches (the first one skips p, q and x)
     const int atag = first ? -1 : SDC_PROF_APPLY;
     prof_begin(h, atag, s);
@@ -1596,11 +1618,11 @@ int pcg_reliable(sdc_handle_s* h, const double* q, double* u, int ncol, const sd
     if (first) {                                                                               \
       DISPATCH_RG(R, G_, launch(h, (k_apply_pq<ZT, R, true, G>), grid2(l0.nN, ncol, R * G),    \
                                 blk, 0, s, s1, ZP, p_prev, p_out, W.q, (const double*)W.beta,  \
-                                l0.ld, ncol, W.partial, (const int*)W.ctl, K > 1 ? 1 : 0));    \
+                                bin, l0.ld, ncol, pqpart, (const int*)W.ctl, K > 1 ? 1 : 0));  \
     } else {                                                                                   \
       DISPATCH_RG(R, G_, launch(h, (k_apply_pq<ZT, R, false, G>), grid2(l0.nN, ncol, R * G),   \
                                 blk, 0, s, s1, ZP, p_prev, p_out, W.q, (const double*)W.beta,  \
-                                l0.ld, ncol, W.partial, (const int*)W.ctl, K > 1 ? 1 : 0));    \
+                                bin, l0.ld, ncol, pqpart, (const int*)W.ctl, K > 1 ? 1 : 0));  \
     }
     if (zb) {
       SDC_APPLY_PQ(__bf16, (const __bf16*)z16)
@@ -1610,16 +1632,20 @@ int pcg_reliable(sdc_handle_s* h, const double* q, double* u, int ncol, const sd
 #undef SDC_APPLY_PQ
     // algorithmic bytes of the steady state: z (stencil), p_prev and q read, p and q written
     prof_end(h, atag, s, (double)l0.nN * 16 + (double)l0.nN * ncol * (bz + 16.0));
-    launch(h, k_fin_alpha, dim3(ncol), blk, 0, s, (const double*)W.partial, nbx,
-           (const double*)W.rz, W.alpha, (const int*)W.active, stop,
-           W.ahist + (size_t)phi * W.ncap);
+    AlphaIn ain{};
+    double* const ah = W.ahist + (size_t)phi * W.ncap;
+    if (inl)
+      ain = AlphaIn{pqpart, nbx, rz, W.active, ah};
+    else
+      launch(h, k_fin_alpha, dim3(ncol), blk, 0, s, (const double*)W.partial, nbx,
+             (const double*)W.rz, W.alpha, (const int*)W.active, stop, ah);
     prof_begin(h, SDC_PROF_UPDATE, s);
     if (r16)
       launch(h, k_update_r4<true, kUpdChunks>, gupd, blk, 0, s, W.r, (const float*)W.q,
-             (const double*)W.alpha, l0.ld, l0.nN, W.partial, r16, stop);
+             (const double*)W.alpha, ain, l0.ld, l0.nN, W.partial, r16, stop);
     else
       launch(h, k_update_r4<false, kUpdChunks>, gupd, blk, 0, s, W.r, (const float*)W.q,
-             (const double*)W.alpha, l0.ld, l0.nN, W.partial, r16, stop);
+             (const double*)W.alpha, ain, l0.ld, l0.nN, W.partial, r16, stop);
     prof_end(h, SDC_PROF_UPDATE, s, (double)l0.nN * ncol * (r16 ? 14 : 12));
     launch(h, k_norm_decide, dim3(1), dim3(SDC_FIN_THREADS), 0, s, (const double*)W.partial,
            gupd.x, W.rr, W.ctl, (const double*)W.aux, (const double*)W.rmax,
