@@ -1904,9 +1904,10 @@ int sdc_create(const sdc_mesh_desc* d, sdc_handle* out) {
   }
   fill_level_dims(l0);
   h->L.push_back(l0);
-  // coarsest level: at most 64 nodes by default (its dense inverse is rebuilt by one work-group
-  // at every sdc_set_sigma: 19 us for some 60 nodes)
-  const uint32_t cmax = d->coarse_max > 0 ? (uint32_t)d->coarse_max : 64u;
+  // coarsest level: at most 128 nodes by default (what k_coarse_inverse takes).  With 64 the
+  // levels of 65..128 nodes cost a cycle 12,000 clocks per visit in the coarse tail for 2,500 of
+  // a larger dense level: 22,050 nodes x 20 columns 1,271 us per solve, 1,242 with 128.
+  const uint32_t cmax = d->coarse_max > 0 ? (uint32_t)d->coarse_max : (uint32_t)SDC_CINV_MAX;
   double hmin = 1e300;
   for (int a = 0; a < 3; ++a)
     for (double v : *w[a]) hmin = std::min(hmin, v);
