@@ -1095,8 +1095,11 @@ __global__ __launch_bounds__(SDC_BLOCK) void k_update_r4(float* __restrict__ r,
   }
   double a;
   if (in.part) {
+    // device-scope loads: their addresses are uniform, and a scalar cache may hold old lines
+    const double rz = ld_flag(in.rz + c);
+    const int act = ld_flag(in.active + c);
     const double pq = block_sum(in.part + (size_t)c * in.nb, in.nb);
-    a = in.active[c] && pq > 0.0 ? in.rz[c] / pq : 0.0;
+    a = act && pq > 0.0 ? rz / pq : 0.0;
     if (blockIdx.x == 0 && threadIdx.x == 0) in.ahist[c] = a;
   } else {
     a = alpha[c];
