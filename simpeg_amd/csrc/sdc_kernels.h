@@ -961,17 +961,19 @@ __device__ __forceinline__ double block_sum(const double* __restrict__ part, uin
 // into u (fp64) by k_ir_fold_ring, so no fp32 iterate is read and written every step.
 // FIRST: p = z, q = A z.  check_stop: return at once when ctl[STOP] is set (only needed when
 // several iterations run between host reads of the stop flag).
-// With in.part every work-group sums its columns' r.z partials itself (k_fin_beta otherwise),
-// while its stencil loads are under way; the first one of a column group also stores r.z.
+// INL: every work-group sums its columns' r.z partials itself (k_fin_beta otherwise), while its
+// stencil loads are under way; the first one of a column group also stores r.z.  (A template
+// argument: with the choice made in the kernel, large levels lost 9 %, 435 -> 474 us per launch
+// on 932,137 nodes x 128 columns.)
 struct BetaIn {
-  const double* part;     // r.z partials, nb per column (null: beta holds the result)
+  const double* part;     // r.z partials, nb per column
   uint32_t nb;
   const double* rz_prev;  // r.z of the previous iteration
   double* rz;             // r.z of this one
   const int* active;
 };
 
-template <typename Z, int R, bool FIRST, int G = 1>
+template <typename Z, int R, bool FIRST, bool INL, int G = 1>
 __global__ __launch_bounds__(SDC_BLOCK) void k_apply_pq(Sten<float> sa, const Z* __restrict__ z,
                                                         const float* __restrict__ p_prev,
                                                         float* __restrict__ p_out,
@@ -983,25 +985,6 @@ __global__ __launch_bounds__(SDC_BLOCK) void k_apply_pq(Sten<float> sa, const Z*
                                                         int check_stop) {
   if (check_stop && ld_flag(ctl + SDC_CTL_STOP)) return;
   SDC_NODE_PROLOGUE_C(sa.nN, sa.remap, R * G)
-  __shared__ double sbeta[R * G];
-  // wavefront w: the columns c0 + w, c0 + w + 4, ...
-  auto sum_beta = [&] {
-    const int lane = threadIdx.x & 63;
-    for (int k = (int)threadIdx.x >> 6; k < R * G; k += SDC_BLOCK / 64) {
-      const int c = min(c0 + k, ncol - 1);
-      double v = 0.0;
-      for (uint32_t b = lane; b < in.nb; b += 64) v += in.part[(size_t)c * in.nb + b];
-#pragma unroll
-      for (int off = 32; off > 0; off >>= 1) v += __shfl_xor(v, off, 64);
-      if (lane == 0) {
-        const double old = FIRST ? 0.0 : in.rz_prev[c];
-        sbeta[k] = !FIRST && in.active[c] && old != 0.0 ? v / old : 0.0;
-        if (bx == 0 && c0 + k < ncol) in.rz[c] = v;
-      }
-    }
-    __syncthreads();
-  };
-  auto beta_of = [&](int k) -> float { return (float)(in.part ? sbeta[k] : beta[c0 + k]); };
   double acc[R * G];
 #pragma unroll
   for (int r = 0; r < R * G; ++r) acc[r] = 0.0;
@@ -1018,14 +1001,14 @@ __global__ __launch_bounds__(SDC_BLOCK) void k_apply_pq(Sten<float> sa, const Z*
     }
     stencil_cols<float, R>(c, z, n, ld, cg, ncol, zc, az);
   };
-  auto finish = [&](int cg, int k0) {
+  auto finish = [&](int cg, int k0, auto beta_of) {
 #pragma unroll
     for (int r = 0; r < R; ++r) {
       if (cg + r < ncol) {
         const size_t o = (size_t)(cg + r) * ld + n;
         float pn = zc[r], qn = az[r];
         if (!FIRST) {
-          const float be = beta_of(k0 + r);
+          const float be = (float)beta_of(k0 + r);
           pn += be * po[r];
           qn += be * qo[r];
         }
@@ -1035,26 +1018,46 @@ __global__ __launch_bounds__(SDC_BLOCK) void k_apply_pq(Sten<float> sa, const Z*
       }
     }
   };
-  if constexpr (G == 1) {
-    if (live) {
+  auto groups = [&](auto beta_of) {
+    if (!live) return;
+    c = node_coef(sten_col(sa, c0), n);
+#pragma unroll 2
+    for (int gq = 0; gq < G; ++gq) {
+      const int cg = c0 + gq * R;
+      if (cg >= ncol) break;
+      if (G > 1 && gq > 0 && set_changes(sa, cg, cg - R)) c = node_coef(sten_col(sa, cg), n);
+      load(cg);
+      finish(cg, gq * R, beta_of);
+    }
+  };
+  if constexpr (INL) {
+    __shared__ double sbeta[R * G];
+    auto mine = [&](int k) { return sbeta[k]; };
+    if (G == 1 && live) {
       c = node_coef(sten_col(sa, c0), n);
       load(c0);
     }
-    if (in.part) sum_beta();
-    if (live) finish(c0, 0);
-  } else {
-    if (in.part) sum_beta();
-    if (live) {
-      c = node_coef(sten_col(sa, c0), n);
-#pragma unroll 2
-      for (int gq = 0; gq < G; ++gq) {
-        const int cg = c0 + gq * R;
-        if (cg >= ncol) break;
-        if (gq > 0 && set_changes(sa, cg, cg - R)) c = node_coef(sten_col(sa, cg), n);
-        load(cg);
-        finish(cg, gq * R);
+    // wavefront w: the columns c0 + w, c0 + w + 4, ...
+    const int lane = threadIdx.x & 63;
+    for (int k = (int)threadIdx.x >> 6; k < R * G; k += SDC_BLOCK / 64) {
+      const int col = min(c0 + k, ncol - 1);
+      double v = 0.0;
+      for (uint32_t b = lane; b < in.nb; b += 64) v += in.part[(size_t)col * in.nb + b];
+#pragma unroll
+      for (int off = 32; off > 0; off >>= 1) v += __shfl_xor(v, off, 64);
+      if (lane == 0) {
+        const double old = FIRST ? 0.0 : in.rz_prev[col];
+        sbeta[k] = !FIRST && in.active[col] && old != 0.0 ? v / old : 0.0;
+        if (bx == 0 && c0 + k < ncol) in.rz[col] = v;
       }
     }
+    __syncthreads();
+    if (G > 1)
+      groups(mine);
+    else if (live)
+      finish(c0, 0, mine);
+  } else {
+    groups([&](int k) { return beta[c0 + k]; });
   }
   block_partials<R * G>(acc, partial, c0, ncol, nbx, bx);
 }
@@ -1062,17 +1065,17 @@ __global__ __launch_bounds__(SDC_BLOCK) void k_apply_pq(Sten<float> sa, const Z*
 // r -= alpha q and per-column |r|^2 partials: a work-group takes CH chunks of SDC_NODES4 nodes
 // (4 per work-item and chunk, all loads issued before the arithmetic), one partial per
 // work-group, so that the single-work-group decision sums few partials per column
-// (R16: also write a bfloat16 copy of r, the multigrid input).  With in.part every work-group
+// (R16: also write a bfloat16 copy of r, the multigrid input).  INL: every work-group
 // sums its column's p.q partials itself (k_fin_alpha otherwise); the first one stores alpha.
 struct AlphaIn {
-  const double* part;  // p.q partials, nb per column (null: alpha holds the result)
+  const double* part;  // p.q partials, nb per column
   uint32_t nb;
   const double* rz;
   const int* active;
   double* ahist;       // alpha out (the ring slot's)
 };
 
-template <bool R16, int CH>
+template <bool R16, int CH, bool INL>
 __global__ __launch_bounds__(SDC_BLOCK) void k_update_r4(float* __restrict__ r,
                                                          const float* __restrict__ q,
                                                          const double* __restrict__ alpha,
@@ -1094,7 +1097,7 @@ __global__ __launch_bounds__(SDC_BLOCK) void k_update_r4(float* __restrict__ r,
     }
   }
   double a;
-  if (in.part) {
+  if (INL) {
     // device-scope loads: their addresses are uniform, and a scalar cache may hold old lines
     const double rz = ld_flag(in.rz + c);
     const int act = ld_flag(in.active + c);

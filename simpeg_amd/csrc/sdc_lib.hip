@@ -1614,21 +1614,26 @@ int pcg_reliable(sdc_handle_s* h, const double* q, double* u, int ncol, const sd
     // the class covers the steady-state launches (the first one skips p, q and x)
     const int atag = first ? -1 : SDC_PROF_APPLY;
     prof_begin(h, atag, s);
-#define SDC_APPLY_PQ(ZT, ZP)                                                                   \
-    if (first) {                                                                               \
-      DISPATCH_RG(R, G_, launch(h, (k_apply_pq<ZT, R, true, G>), grid2(l0.nN, ncol, R * G),    \
-                                blk, 0, s, s1, ZP, p_prev, p_out, W.q, (const double*)W.beta,  \
-                                bin, l0.ld, ncol, pqpart, (const int*)W.ctl, K > 1 ? 1 : 0));  \
-    } else {                                                                                   \
-      DISPATCH_RG(R, G_, launch(h, (k_apply_pq<ZT, R, false, G>), grid2(l0.nN, ncol, R * G),   \
-                                blk, 0, s, s1, ZP, p_prev, p_out, W.q, (const double*)W.beta,  \
-                                bin, l0.ld, ncol, pqpart, (const int*)W.ctl, K > 1 ? 1 : 0));  \
+#define SDC_APPLY_PQ(ZT, ZP, FIRST, INL)                                                       \
+    DISPATCH_RG(R, G_, launch(h, (k_apply_pq<ZT, R, FIRST, INL, G>), grid2(l0.nN, ncol, R * G), \
+                              blk, 0, s, s1, ZP, p_prev, p_out, W.q, (const double*)W.beta,    \
+                              bin, l0.ld, ncol, pqpart, (const int*)W.ctl, K > 1 ? 1 : 0))
+#define SDC_APPLY_PQ_Z(ZT, ZP)            \
+    if (first && inl) {                   \
+      SDC_APPLY_PQ(ZT, ZP, true, true);   \
+    } else if (first) {                   \
+      SDC_APPLY_PQ(ZT, ZP, true, false);  \
+    } else if (inl) {                     \
+      SDC_APPLY_PQ(ZT, ZP, false, true);  \
+    } else {                              \
+      SDC_APPLY_PQ(ZT, ZP, false, false); \
     }
     if (zb) {
-      SDC_APPLY_PQ(__bf16, (const __bf16*)z16)
+      SDC_APPLY_PQ_Z(__bf16, (const __bf16*)z16)
     } else {
-      SDC_APPLY_PQ(float, (const float*)W.z)
+      SDC_APPLY_PQ_Z(float, (const float*)W.z)
     }
+#undef SDC_APPLY_PQ_Z
 #undef SDC_APPLY_PQ
     // algorithmic bytes of the steady state: z (stencil), p_prev and q read, p and q written
     prof_end(h, atag, s, (double)l0.nN * 16 + (double)l0.nN * ncol * (bz + 16.0));
@@ -1640,12 +1645,18 @@ int pcg_reliable(sdc_handle_s* h, const double* q, double* u, int ncol, const sd
       launch(h, k_fin_alpha, dim3(ncol), blk, 0, s, (const double*)W.partial, nbx,
              (const double*)W.rz, W.alpha, (const int*)W.active, stop, ah);
     prof_begin(h, SDC_PROF_UPDATE, s);
-    if (r16)
-      launch(h, k_update_r4<true, kUpdChunks>, gupd, blk, 0, s, W.r, (const float*)W.q,
-             (const double*)W.alpha, ain, l0.ld, l0.nN, W.partial, r16, stop);
+#define SDC_UPDATE_R(R16, INL)                                                              \
+    launch(h, (k_update_r4<R16, kUpdChunks, INL>), gupd, blk, 0, s, W.r, (const float*)W.q,  \
+           (const double*)W.alpha, ain, l0.ld, l0.nN, W.partial, r16, stop)
+    if (r16 && inl)
+      SDC_UPDATE_R(true, true);
+    else if (r16)
+      SDC_UPDATE_R(true, false);
+    else if (inl)
+      SDC_UPDATE_R(false, true);
     else
-      launch(h, k_update_r4<false, kUpdChunks>, gupd, blk, 0, s, W.r, (const float*)W.q,
-             (const double*)W.alpha, ain, l0.ld, l0.nN, W.partial, r16, stop);
+      SDC_UPDATE_R(false, false);
+#undef SDC_UPDATE_R
     prof_end(h, SDC_PROF_UPDATE, s, (double)l0.nN * ncol * (r16 ? 14 : 12));
     launch(h, k_norm_decide, dim3(1), dim3(SDC_FIN_THREADS), 0, s, (const double*)W.partial,
            gupd.x, W.rr, W.ctl, (const double*)W.aux, (const double*)W.rmax,
