@@ -664,14 +664,22 @@ int tail_npt(uint32_t nN) {
   return nN <= 2 * SDC_TAIL_THREADS ? 2 : nN <= 4 * SDC_TAIL_THREADS ? 4 : 8;
 }
 
-// W-cycle level: the requested one, or (wcycle_level = -1) the first level with at most 1/4 of
-// the finest level's nodes (level 1 unless the first coarsening step only touched a small core
-// of a padded mesh) -- a second visit there costs ~15 % of a cycle and removes an iteration on
-// padded meshes with strong contrasts.  Never the coarsest level.
+// W-cycle level: the requested one, or (wcycle_level = -1) on large meshes the first level with at
+// most 1/4 of the finest level's nodes (level 1 unless the first coarsening step only touched a
+// small core of a padded mesh) -- a second visit there costs ~15 % of a cycle and removes an
+// iteration or two on padded meshes.  On smaller meshes the coarse levels cost the latency of
+// their launches and steps, not bandwidth, and the second visit 20-30 % of a cycle, more than the
+// iterations it saves.  Time of a V-cycle solve over a W one, Robin boundaries: 2,550..209,440
+// nodes 0.73 to 1.01 (18 cases, mean 0.91: 9 iterations stay 9 or become 10 or 11, 15 layered ones
+// 19), 669,120 nodes x 26 columns 1.03, 932,137 x 128 1.035.  Neumann operators keep the W step: the
+// V-cycle leaves more of the nearly free constant in the error at the same residual (1.9e-9
+// against 1e-10 or less).  Never the coarsest level.
+constexpr uint32_t kWcycleNodes = 1u << 18;
 int pick_wlevel(const sdc_handle_s* h) {
   const int nl = (int)h->L.size();
   int l = h->prm.wcycle_level;
   if (l < 0) {
+    if (h->bc != SDC_BC_NEUMANN && h->L[0].nN < kWcycleNodes) return 0;
     l = 0;
     for (int k = 1; k < nl - 1; ++k)
       if ((size_t)h->L[k].nN * 4 <= (size_t)h->L[0].nN) {
@@ -685,8 +693,7 @@ int pick_wlevel(const sdc_handle_s* h) {
 // The coarse tail that one work-group per column runs (sdc_tail.h): from the first level with at
 // most SDC_TAIL_NODES nodes whose cycle fits into 160 KB of LDS on, with at least one level above
 // the coarsest.  The finest level may be that one, unless it reads a bf16 residual (storage 3,
-// 4) or smooths another number of steps than the coarser ones.  On the 22,050-node block model the tail then starts at the W level (6,348 nodes), which
-// took 14 launches before.
+// 4) or smooths another number of steps than the coarser ones.
 // at0 = false keeps the finest level out as well (sdc_vcycle, whose finest level shows the storage
 // it was asked for).
 void pick_tail(sdc_handle_s* h, bool at0 = true) {
