@@ -259,6 +259,7 @@ struct sdc_handle_s {
   sdc_params prm;
   int vstore = 1;  // storage of the fp32 V-cycle vectors in this call (as sdc_params.vcycle_bf16)
   int wlevel = 0;  // level whose coarse correction runs twice (0: none)
+  int wnow = 0;    // the same for the current call (solve_wlevel)
   // single-launch coarse tail: its first level (-1: none), its descriptor, the operator image of
   // every set (tail_img_cap floats) and the tables; tail_stale: the image does not belong to the
   // current operator or plan (ensure_tail)
@@ -690,6 +691,20 @@ int pick_wlevel(const sdc_handle_s* h) {
   return (l >= 1 && l < nl - 1) ? l : 0;
 }
 
+// The same for a solve of ncol columns: with few columns the coarse levels of a large mesh, too,
+// cost latency.  Only where the W level runs as launches (the tail's steps are fixed when the
+// operator is set).  Time of a V-cycle solve over a W one on 932,137 nodes, random-field and
+// layered model: 1 column 0.80 and 0.88, 3 0.84 and 0.93, 6 0.87 and 0.97, 9 0.90 and 1.00, 16 0.92
+// and 1.02, 48 0.98 and 1.09 (10 iterations for 9, and 15 for 12).
+constexpr size_t kWcycleColumns = (size_t)8 << 20;  // nodes x columns
+int solve_wlevel(const sdc_handle_s* h, int ncol) {
+  const bool launched = h->tail_level < 0 || h->wlevel < h->tail_level;
+  if (h->prm.wcycle_level < 0 && h->bc != SDC_BC_NEUMANN && launched &&
+      (size_t)h->L[0].nN * (size_t)ncol < kWcycleColumns)
+    return 0;
+  return h->wlevel;
+}
+
 // The coarse tail that one work-group per column runs (sdc_tail.h): from the first level with at
 // most SDC_TAIL_NODES nodes whose cycle fits into 160 KB of LDS on, with at least one level above
 // the coarsest.  The finest level may be that one, unless it reads a bf16 residual (storage 3,
@@ -1074,7 +1089,7 @@ int vcycle(sdc_handle_s* h, int l, const B* b, O* x, int ncol, bool dot_out, con
   constexpr bool sep = !std::is_same<O, S>::value;
   // W-cycle step on one level: the coarse correction runs twice, with nu_post smoothing steps
   // between the two (the error propagator stays symmetric: S* C S C S)
-  const int ngam = (h->wlevel > 0 && l == h->wlevel) ? 2 : 1;
+  const int ngam = (h->wnow > 0 && l == h->wnow) ? 2 : 1;
   // smoothing steps between the two coarse corrections of a W step (any number keeps the cycle
   // symmetric: every Chebyshev polynomial in D^-1 A is self-adjoint in the A inner product)
   const int num = h->prm.wcycle_smooth > 0 ? h->prm.wcycle_smooth : nu2;
@@ -1318,6 +1333,7 @@ int graph_run(sdc_handle_s* h, const void* b, void* x, int ncol, int variant, hi
   if (!h->prm.graph || (h->prof_mask & vcycle_tags)) return fn(st);
   // kernels recorded in operator-set mode carry the column -> set map
   if (h->cur_cset) variant |= 1 << 24;
+  if (h->wnow != h->wlevel) variant |= 1 << 25;
   for (const auto& g : h->graphs)
     if (g.b == b && g.x == x && g.ncol == ncol && g.variant == variant) {
       HIPCK(hipGraphLaunch(g.exec, st));
@@ -2210,6 +2226,7 @@ int sdc_vcycle(sdc_handle h, int dtype, const void* b, void* z, int ncol, void* 
   if (!h->sigma_set) return fail(SDC_ERR_STATE, "no operator set: call sdc_set_sigma or sdc_set_coefficients first");
   DeviceGuard dg(h->device);
   hipStream_t st = (hipStream_t)stream;
+  h->wnow = h->wlevel;
   if (dtype == SDC_F64) {
     CK(ensure_work<double>(h, ncol));
     CK(vcycle0<double>(h, (const double*)b, (double*)z, ncol, false, nullptr, st));
@@ -2238,6 +2255,7 @@ int sdc_solve(sdc_handle h, const double* q, double* u, int ncol, const sdc_solv
     return fail(SDC_ERR_ARG, "mixed mode needs inner_tol > 0 and max_outer >= 1");
   DeviceGuard dg(h->device);
   hipStream_t st = (hipStream_t)stream;
+  h->wnow = solve_wlevel(h, ncol);
   const Level& l0 = h->L[0];
   const int R = pick_r(h, ncol, h->L[0].nN);
   const dim3 g = grid2(l0.nN, ncol, R);

@@ -44,3 +44,26 @@ def test_w_step_in_the_tail(gpu, shape, level):
     out = eng.from_block(eng.vcycle(eng.to_block(a, torch.float32)).double())
     assert rel(out, ref) < 1e-5
     eng.close()
+
+
+def test_columns_choose_the_cycle_of_a_solve(gpu):
+    """Few columns on a large mesh take the V-cycle, many the W-cycle, whatever was solved and
+    recorded before: the potentials are those of the explicit levels."""
+    from simpeg_amd.engine import NodalEngine
+
+    rng = np.random.default_rng(4)
+    eng = NodalEngine([np.full(63, 10.0)] * 3, np.zeros(3))
+    eng.set_sigma(np.exp(0.5 * rng.standard_normal(eng.nC)) * 0.01)
+    q = eng.to_block(rng.standard_normal((eng.nN, 33)))
+    cases = {3: 0, 31: 0, 33: 1}  # 2^18 nodes x 32 columns = 2^23
+    ref = {}
+    for n, level in cases.items():
+        eng.set_params(wcycle_level=level)
+        ref[n] = eng.solve(q[:n].contiguous(), n)
+    eng.set_params(wcycle_level=-1)
+    for _ in range(2):
+        for n in cases:
+            u, r = eng.solve(q[:n].contiguous(), n)
+            assert r.converged and r.iters == ref[n][1].iters
+            assert torch.equal(u, ref[n][0]), n
+    eng.close()
