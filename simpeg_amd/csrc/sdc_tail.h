@@ -37,9 +37,9 @@ struct TailLev {
 };
 
 // Transfer between level l and l + 1: strides of the grids, the LDS offset of its table (two
-// words per coarse node, tail_table_entry; the top level's is read from global memory) and where its interpolation weights start (Xfer::wx,
-// wy, wz one after the other): LDS offset w.  The top level's weights are laid out per coarse node
-// in the image instead (SDC_TAIL_WR for the restriction, SDC_TAIL_WP for the interpolation, each
+// words per coarse node, tail_table_entry; the top level's is read from global memory) and where
+// its interpolation weights start (Xfer::wx, wy, wz one after the other): LDS offset w.  The top
+// level's weights are laid out per coarse node in the image instead (SDC_TAIL_WR for the restriction, SDC_TAIL_WP for the interpolation, each
 // an array over the coarse nodes): read from L2 point by point, 9 gathers of stride 2 per
 // work-item, they took 20,000 of a launch's 77,000 clocks on 7,406 + 1,352 nodes.
 #define SDC_TAIL_WR 27
