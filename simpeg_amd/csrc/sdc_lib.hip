@@ -2287,8 +2287,8 @@ int sdc_solve(sdc_handle h, const double* q, double* u, int ncol, const sdc_solv
     S.max_rel_res = m;
     return SDC_OK;
   };
-  // plain fp64 PCG from u = 0
-  auto fp64_solve = [&](int* iters) -> int {
+  // plain fp64 PCG from u = 0 towards the residual `aim`
+  auto fp64_solve = [&](double aim, int* iters) -> int {
     CK(ensure_work<double>(h, ncol));
     Work<double>& W = h->w64;
     hipLaunchKernelGGL(k_zero<unsigned>, dim3(nblk(l0.nN)), blk, 0, st, W.qmask, (size_t)l0.nN);
@@ -2297,7 +2297,7 @@ int sdc_solve(sdc_handle h, const double* q, double* u, int ncol, const sdc_solv
                                      (__bf16*)nullptr, (const int*)nullptr, (const double* const*)nullptr));
     hipLaunchKernelGGL(k_fin_norm, dim3(ncol), blk, 0, st, (const double*)W.partial, nbx, W.aux,
                        W.active, 0, (const int*)nullptr);
-    CK(pcg<double>(h, u, ncol, o->tol, o->max_iter, nullptr, iters, st));
+    CK(pcg<double>(h, u, ncol, aim, o->max_iter, nullptr, iters, st));
     S.outer = 1;
     DISPATCH_R(R, hipLaunchKernelGGL((k_ir_residual<double, R, false>), g, blk, 0, st, s2, q,
                                      (const double*)u, W.z, l0.ld, ncol, pf, W.partial,
@@ -2305,16 +2305,17 @@ int sdc_solve(sdc_handle h, const double* q, double* u, int ncol, const sdc_solv
     hipLaunchKernelGGL(k_fin_norm, dim3(ncol), blk, 0, st, (const double*)W.partial, nbx, W.orr,
                        W.active, 0, (const int*)nullptr);
     CK(rel_max(W.orr, W.aux));
-    // converged when every column met the PCG test (recursive residual)
+    // converged when every column met the PCG test (recursive residual), or, short of an aim
+    // below the tolerance, when the true residual met the tolerance
     HIPCK(hipMemcpyAsync(h->h_flag, W.counters + 2, sizeof(int), hipMemcpyDeviceToHost, st));
     HIPCK(hipStreamSynchronize(st));
-    S.converged = (h->h_flag[0] == 0) ? 1 : 0;
+    S.converged = (h->h_flag[0] == 0 || (aim < o->tol && S.max_rel_res <= o->tol)) ? 1 : 0;
     return SDC_OK;
   };
   if (o->mode == SDC_MODE_MIXED && h->mixed_stalled) {
-    // an earlier mixed solve on this operator stalled: fp64 from the start
+    // an earlier mixed solve on this operator stalled: fp64 from the start, to the same residual
     int it = 0;
-    CK(fp64_solve(&it));
+    CK(fp64_solve(mixed_aim(h, o->tol), &it));
     S.fp64_iters = it;
   } else if (o->mode == SDC_MODE_MIXED) {
     CK(pcg_reliable(h, q, u, ncol, o, S, st));
@@ -2346,7 +2347,7 @@ int sdc_solve(sdc_handle h, const double* q, double* u, int ncol, const sdc_solv
     }
   } else if (o->mode == SDC_MODE_FP64) {
     int it = 0;
-    CK(fp64_solve(&it));
+    CK(fp64_solve(o->tol, &it));
     S.iters = it;
   } else {
     h->vstore = h->prm.vcycle_bf16;
