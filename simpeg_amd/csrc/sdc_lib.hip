@@ -2350,7 +2350,7 @@ int sdc_solve(sdc_handle h, const double* q, double* u, int ncol, const sdc_solv
     CK(fp64_solve(o->tol, &it));
     S.iters = it;
   } else {
-    h->vstore = h->prm.vcycle_bf16;
+    h->vstore = mixed_storage(h);
     CK(ensure_work<float>(h, ncol));
     CK(ensure_tail(h, st));
     Work<float>& W = h->w32;
@@ -2363,7 +2363,10 @@ int sdc_solve(sdc_handle h, const double* q, double* u, int ncol, const sdc_solv
                        W.active, 0, (const int*)nullptr);
     hipLaunchKernelGGL(k_fin_norm, dim3(ncol), blk, 0, st, (const double*)W.partial, nbx, W.orr,
                        W.active, 0, (const int*)nullptr);
-    const double tol2 = o->tol * o->tol;
+    // Every refinement gains inner_tol; one that only has to get from the tolerance to an aim below
+    // it gains what that takes, and none follows one that gained nothing below the tolerance.
+    const double aim = mixed_aim(h, o->tol), tol2 = aim * aim;
+    double inner = o->inner_tol, last = INFINITY;
     for (int outer = 0;; ++outer) {
       if (outer > 0) {
         prof_begin(h, SDC_PROF_REFINE, st);
@@ -2381,13 +2384,14 @@ int sdc_solve(sdc_handle h, const double* q, double* u, int ncol, const sdc_solv
       CK(rel_max(W.orr, W.aux));
       const int open = h->h_flag[0];
       S.outer = outer;
-      if (open == 0) {
-        S.converged = 1;
-        break;
-      }
+      const bool met = aim < o->tol && S.max_rel_res <= o->tol;
+      S.converged = open == 0 || met;
+      if (open == 0 || (met && S.max_rel_res > 0.5 * last)) break;
+      if (met) inner = std::min(0.5, std::max(o->inner_tol, 0.5 * aim / S.max_rel_res));
+      last = S.max_rel_res;
       if (outer == o->max_outer) break;
       int it = 0;
-      CK(pcg<float>(h, W.x, ncol, o->inner_tol, o->max_iter, W.omask, &it, st));
+      CK(pcg<float>(h, W.x, ncol, inner, o->max_iter, W.omask, &it, st));
       S.iters += it;
       DISPATCH_R(R, hipLaunchKernelGGL((k_ir_update<float, R>), g, blk, 0, st, u, (const float*)W.x,
                                        l0.ld, l0.nN, ncol));

@@ -36,3 +36,15 @@ def test_solves_after_a_stalled_one(gpu, npad, seed):
     assert r.converged and r.iters == 0 and r.fp64_iters > 0, r  # fp64 from the start
     assert r.max_rel_res <= 1.01 * TOL / 32, r
     assert rel(u[:n, :eng.nN].cpu().numpy(), ref) < 1e-9
+
+
+@pytest.mark.parametrize("npad", [3, 4, 6])
+@pytest.mark.parametrize("seed", [0, 1])
+def test_iterative_refinement(gpu, npad, seed):
+    eng, q, n, ref = _problem(npad, seed)
+    _, r64 = eng.solve(q, n, mode="fp64", tol=TOL)
+    u, r = eng.solve(q, n, mode="mixed_ir", tol=TOL)
+    print(r64, r)
+    assert r.converged and r.max_rel_res <= TOL / 32, r
+    assert r.iters <= 2 * r64.iters, (r, r64)
+    assert rel(u[:n, :eng.nN].cpu().numpy(), ref) < 1e-9
