@@ -665,44 +665,53 @@ int tail_npt(uint32_t nN) {
   return nN <= 2 * SDC_TAIL_THREADS ? 2 : nN <= 4 * SDC_TAIL_THREADS ? 4 : 8;
 }
 
-// W-cycle level: the requested one, or (wcycle_level = -1) on large meshes the first level with at
-// most 1/4 of the finest level's nodes (level 1 unless the first coarsening step only touched a
-// small core of a padded mesh) -- a second visit there costs ~15 % of a cycle and removes an
-// iteration or two on padded meshes.  On smaller meshes the coarse levels cost the latency of
-// their launches and steps, not bandwidth, and the second visit 20-30 % of a cycle, more than the
-// iterations it saves.  Time of a V-cycle solve over a W one, Robin boundaries: 2,550..209,440
-// nodes 0.73 to 1.01 (18 cases, mean 0.91: 9 iterations stay 9 or become 10 or 11, 15 layered ones
-// 19), 669,120 nodes x 26 columns 1.03, 932,137 x 128 1.035.  Neumann operators keep the W step: the
-// V-cycle leaves more of the nearly free constant in the error at the same residual (1.9e-9
-// against 1e-10 or less).  Never the coarsest level.
+// The first level with at most 1/4 of the finest level's nodes (level 1 unless the first coarsening
+// step only touched a small core of a padded mesh), never the coarsest (0: none).
+int quarter_level(const sdc_handle_s* h) {
+  for (int k = 1; k < (int)h->L.size() - 1; ++k)
+    if ((size_t)h->L[k].nN * 4 <= (size_t)h->L[0].nN) return k;
+  return 0;
+}
+
+// W-cycle level of the handle: the requested one, or (wcycle_level = -1) quarter_level on Neumann
+// operators and on large meshes, where a second visit there costs ~15 % of a cycle and removes
+// an iteration or two on padded meshes; elsewhere none.  Never the coarsest level.  Neumann
+// operators keep the W step: the V-cycle leaves more of the nearly free constant in the error at
+// the same residual (1.9e-9 against 1e-10 or less).
 constexpr uint32_t kWcycleNodes = 1u << 18;
 int pick_wlevel(const sdc_handle_s* h) {
   const int nl = (int)h->L.size();
   int l = h->prm.wcycle_level;
   if (l < 0) {
     if (h->bc != SDC_BC_NEUMANN && h->L[0].nN < kWcycleNodes) return 0;
-    l = 0;
-    for (int k = 1; k < nl - 1; ++k)
-      if ((size_t)h->L[k].nN * 4 <= (size_t)h->L[0].nN) {
-        l = k;
-        break;
-      }
+    l = quarter_level(h);
   }
   return (l >= 1 && l < nl - 1) ? l : 0;
 }
 
-// The same for a solve of ncol columns: with few columns the coarse levels of a large mesh, too,
-// cost latency.  Only where the W level runs as launches (the tail's steps are fixed when the
-// operator is set).  Time of a V-cycle solve over a W one on 932,137 nodes, random-field and
-// layered model: 1 column 0.80 and 0.88, 3 0.84 and 0.93, 6 0.87 and 0.97, 9 0.90 and 1.00, 16 0.92
-// and 1.02, 48 0.98 and 1.09 (10 iterations for 9, and 15 for 12).
+// The same for a solve of ncol columns on a Robin operator with wcycle_level = -1.  With few
+// columns, and in fp64 on smaller meshes, the coarse levels cost the latency of their launches,
+// not bandwidth, and the second visit 20-30 % of a cycle, more than the iterations it saves, those
+// included that make up for the V-cycle's errors (solve_aim).  Mixed solves on smaller meshes have
+// those levels in the tail, where the second visit is cheap.  Time of a V-cycle solve to its aim
+// over a W one to the tolerance (random-field, block and layered models, means):
+//   nodes x columns    fp64   mixed          nodes x columns    fp64   mixed
+//     2,550 x  4       0.94   1.08           275,655 x  2       0.85   0.90
+//    22,050 x 20       0.90   1.03           275,655 x 24       0.93   1.02
+//    54,675 x 20       0.91   1.02           329,904 x  8       0.84   0.94
+//   106,689 x  4       0.89   0.96           329,904 x 24       0.96   1.03
+//   106,689 x 48       1.04   1.09           932,137 x  3       0.89   0.93
+//   199,080 x  4       0.85   0.91           932,137 x  8       0.97   0.97
+//   199,080 x 48       0.98   1.05         3,289,545 x  2       0.98   0.96
+// (932,137 x 48 mixed, both to the tolerance: 0.98 and 1.09.)  Only where the W level runs as
+// launches.
 constexpr size_t kWcycleColumns = (size_t)8 << 20;  // nodes x columns
-int solve_wlevel(const sdc_handle_s* h, int ncol) {
-  const bool launched = h->tail_level < 0 || h->wlevel < h->tail_level;
-  if (h->prm.wcycle_level < 0 && h->bc != SDC_BC_NEUMANN && launched &&
-      (size_t)h->L[0].nN * (size_t)ncol < kWcycleColumns)
-    return 0;
-  return h->wlevel;
+int solve_wlevel(const sdc_handle_s* h, int ncol, bool fp64) {
+  if (h->prm.wcycle_level >= 0 || h->bc == SDC_BC_NEUMANN) return h->wlevel;
+  const int w = quarter_level(h);
+  if (h->L[0].nN < kWcycleNodes) return fp64 ? 0 : w;
+  const bool launched = h->tail_level < 0 || w < h->tail_level;
+  return launched && (size_t)h->L[0].nN * (size_t)ncol < kWcycleColumns ? 0 : w;
 }
 
 // The coarse tail that one work-group per column runs (sdc_tail.h): from the first level with at
@@ -782,38 +791,6 @@ void pick_tail(sdc_handle_s* h, bool at0 = true) {
     const TailXf& x0 = d.xf[0];
     d.imgs = 8 * (size_t)tail_npt(d.lv[0].nN) * SDC_TAIL_THREADS + d.nimg +
              up4((size_t)(SDC_TAIL_WR + SDC_TAIL_WP) * x0.cN);
-    // the cycle: down to the W level once, its coarse correction twice (once without a W level)
-    const int w = h->wlevel >= lt && h->wlevel > 0 ? h->wlevel - lt : -1;
-    const int last = nlev - 1;
-    auto step = [&](TailOp op, int l) {
-      d.op[d.nop] = op;
-      d.lev[d.nop++] = (uint8_t)l;
-    };
-    for (int l = 0; l < w; ++l) {
-      step(TAIL_PRE, l);
-      step(TAIL_DOWN, l);
-    }
-    if (w >= 0) step(TAIL_PRE, w);
-    for (int gam = 0; gam < (w >= 0 ? 2 : 1); ++gam) {
-      if (w >= 0) step(TAIL_DOWN, w);
-      for (int l = w + 1; l < last; ++l) {
-        step(TAIL_PRE, l);
-        step(TAIL_DOWN, l);
-      }
-      step(TAIL_DENSE, last);
-      for (int l = last - 1; l > w; --l) {
-        step(TAIL_UP, l);
-        step(TAIL_POST, l);
-      }
-      if (w >= 0) {
-        step(TAIL_UP, w);
-        step(gam == 0 ? TAIL_MID : TAIL_POST, w);
-      }
-    }
-    for (int l = w - 1; l >= 0; --l) {
-      step(TAIL_UP, l);
-      step(TAIL_POST, l);
-    }
     h->tail = d;
     h->tail_level = lt;
     return;
@@ -1017,6 +994,42 @@ Cheb cheb_coefs(const sdc_params& p) {
   return c;
 }
 
+// The steps of the tail's cycle: down to the W level once, its coarse correction twice (once without
+// a W level in the tail).
+void tail_program(const sdc_handle_s* h, TailDesc& d) {
+  const int w = h->wnow >= h->tail_level && h->wnow > 0 ? h->wnow - h->tail_level : -1;
+  const int last = (int)h->L.size() - 1 - h->tail_level;
+  auto step = [&](TailOp op, int l) {
+    d.op[d.nop] = op;
+    d.lev[d.nop++] = (uint8_t)l;
+  };
+  for (int l = 0; l < w; ++l) {
+    step(TAIL_PRE, l);
+    step(TAIL_DOWN, l);
+  }
+  if (w >= 0) step(TAIL_PRE, w);
+  for (int gam = 0; gam < (w >= 0 ? 2 : 1); ++gam) {
+    if (w >= 0) step(TAIL_DOWN, w);
+    for (int l = w + 1; l < last; ++l) {
+      step(TAIL_PRE, l);
+      step(TAIL_DOWN, l);
+    }
+    step(TAIL_DENSE, last);
+    for (int l = last - 1; l > w; --l) {
+      step(TAIL_UP, l);
+      step(TAIL_POST, l);
+    }
+    if (w >= 0) {
+      step(TAIL_UP, w);
+      step(gam == 0 ? TAIL_MID : TAIL_POST, w);
+    }
+  }
+  for (int l = w - 1; l >= 0; --l) {
+    step(TAIL_UP, l);
+    step(TAIL_POST, l);
+  }
+}
+
 // The cycle of levels tail_level .. L-1 for every column in one launch (one work-group per
 // column); b and x are the tail level's blocks; partial non-null: one b.x per column.
 template <typename B, typename O>
@@ -1024,6 +1037,7 @@ int tail_cycle(sdc_handle_s* h, const B* b, O* x, int ncol, double* partial, con
                hipStream_t st) {
   if (h->tail_stale) return fail(SDC_ERR_STATE, "internal: tail image");
   TailDesc d = h->tail;
+  tail_program(h, d);
   d.cset = h->cur_cset;
   // level 0 smooths nu_pre / nu_post steps, coarser levels nu_coarse where that is set; a tail
   // that holds both has one count for all its levels only if they agree (pick_tail)
@@ -1333,7 +1347,7 @@ int graph_run(sdc_handle_s* h, const void* b, void* x, int ncol, int variant, hi
   if (!h->prm.graph || (h->prof_mask & vcycle_tags)) return fn(st);
   // kernels recorded in operator-set mode carry the column -> set map
   if (h->cur_cset) variant |= 1 << 24;
-  if (h->wnow != h->wlevel) variant |= 1 << 25;
+  variant |= h->wnow << 25;  // and the cycle (at most 32 levels)
   for (const auto& g : h->graphs)
     if (g.b == b && g.x == x && g.ncol == ncol && g.variant == variant) {
       HIPCK(hipGraphLaunch(g.exec, st));
@@ -1485,14 +1499,26 @@ int pcg(sdc_handle_s* h, T* x, int ncol, double tol, int maxit, const int* col_m
   return SDC_OK;
 }
 
-// The residual that a mixed solve works towards.  With Neumann boundaries nothing but the three
-// edges of the grounded corner holds the constant, so a residual's sum shifts all potentials: at
-// 22,000..230,000 nodes (20 solves) the error of u was up to 107 times the relative residual
-// (8.5e-9 at 7.9e-11).  Two iterations more of 10 to 15 take it to 1.5e-10 at the default
-// tolerance.  A solve that ends between the two still has converged, and no solve is asked for
-// less than fp64 sums can show.
-double mixed_aim(const sdc_handle_s* h, double tol) {
-  return h->bc == SDC_BC_NEUMANN ? std::min(tol, std::max(tol / 32, 2e-12)) : tol;
+// The residual that a solve works towards: the tolerance, or less where the error would outgrow
+// the residual.  A solve that ends between the two still has converged, and none is asked for less
+// than the sums of its precision can show.
+// Neumann operators, mixed: nothing but the three edges of the grounded corner holds the constant,
+// so a residual's sum shifts all potentials: at 22,000..230,000 nodes (20 solves) the error of u was
+// up to 107 times the relative residual (8.5e-9 at 7.9e-11).  Two iterations more of 10 to 15 take it
+// to 1.5e-10 at the default tolerance.
+// Robin operators, V-cycle where the mesh has a level for the W step: at the same residual the
+// V-cycle leaves more of the smooth error, and its last iteration passes the tolerance by less.  Over
+// 117 problems (2,550..3,289,545 nodes, 1..48 columns, three kinds of model) the errors of V-cycle
+// solves to the tolerance were 1.3 to 19 times those of W-cycle solves in fp64 (mean per size; at
+// most 115) and 0.6 to 12 times in mixed precision; to the aims here 0.04 to 0.45 (at most 2.7) and
+// 0.08 to 0.64 times.
+double solve_aim(const sdc_handle_s* h, double tol, bool fp64) {
+  double f = 1.0;
+  if (h->bc == SDC_BC_NEUMANN)
+    f = fp64 ? 1.0 : 32.0;
+  else if (h->wnow == 0 && quarter_level(h) > 0)
+    f = fp64 ? 32.0 : 10.0;
+  return std::min(tol, std::max(tol / f, fp64 ? 1e-14 : 2e-12));
 }
 
 // fp32 PCG with reliable updates: the fp32 partial solution is folded into the fp64 solution u
@@ -1536,7 +1562,7 @@ int pcg_reliable(sdc_handle_s* h, const double* q, double* u, int ncol, const sd
   const Sten<double> s2 = make_sten<double>(h, 0, 2);
   Sten<float> s1 = make_sten<float>(h, 0, 1);
   if (s1.remap) s1.remap = kApplyBand;
-  const double aim = mixed_aim(h, o->tol), tol2 = aim * aim;
+  const double aim = solve_aim(h, o->tol, false), tol2 = aim * aim;
   const double delta2 = h->prm.reliable_delta * h->prm.reliable_delta;
   const int maxit = o->max_iter;
   // Stall guard: a reliable update is forced after kStallWindow iterations without one, and the
@@ -2255,7 +2281,7 @@ int sdc_solve(sdc_handle h, const double* q, double* u, int ncol, const sdc_solv
     return fail(SDC_ERR_ARG, "mixed mode needs inner_tol > 0 and max_outer >= 1");
   DeviceGuard dg(h->device);
   hipStream_t st = (hipStream_t)stream;
-  h->wnow = solve_wlevel(h, ncol);
+  h->wnow = solve_wlevel(h, ncol, o->mode == SDC_MODE_FP64);
   const Level& l0 = h->L[0];
   const int R = pick_r(h, ncol, h->L[0].nN);
   const dim3 g = grid2(l0.nN, ncol, R);
@@ -2315,7 +2341,7 @@ int sdc_solve(sdc_handle h, const double* q, double* u, int ncol, const sdc_solv
   if (o->mode == SDC_MODE_MIXED && h->mixed_stalled) {
     // an earlier mixed solve on this operator stalled: fp64 from the start, to the same residual
     int it = 0;
-    CK(fp64_solve(mixed_aim(h, o->tol), &it));
+    CK(fp64_solve(solve_aim(h, o->tol, false), &it));
     S.fp64_iters = it;
   } else if (o->mode == SDC_MODE_MIXED) {
     CK(pcg_reliable(h, q, u, ncol, o, S, st));
@@ -2330,7 +2356,7 @@ int sdc_solve(sdc_handle h, const double* q, double* u, int ncol, const sdc_solv
                                        (const double*)u, W.r, l0.ld, ncol, pf, W.partial,
                                        W32.qmask, (__bf16*)nullptr, (const int*)nullptr, (const double* const*)nullptr));
       const double tin =
-          std::min(0.5, 0.5 * mixed_aim(h, o->tol) / std::max(S.max_rel_res, 1e-300));
+          std::min(0.5, 0.5 * solve_aim(h, o->tol, false) / std::max(S.max_rel_res, 1e-300));
       int it = 0;
       CK(pcg<double>(h, W.x, ncol, tin, o->max_iter, nullptr, &it, st));
       S.fp64_iters = it;
@@ -2347,7 +2373,7 @@ int sdc_solve(sdc_handle h, const double* q, double* u, int ncol, const sdc_solv
     }
   } else if (o->mode == SDC_MODE_FP64) {
     int it = 0;
-    CK(fp64_solve(o->tol, &it));
+    CK(fp64_solve(solve_aim(h, o->tol, true), &it));
     S.iters = it;
   } else {
     h->vstore = mixed_storage(h);
@@ -2365,7 +2391,7 @@ int sdc_solve(sdc_handle h, const double* q, double* u, int ncol, const sdc_solv
                        W.active, 0, (const int*)nullptr);
     // Every refinement gains inner_tol; one that only has to get from the tolerance to an aim below
     // it gains what that takes, and none follows one that gained nothing below the tolerance.
-    const double aim = mixed_aim(h, o->tol), tol2 = aim * aim;
+    const double aim = solve_aim(h, o->tol, false), tol2 = aim * aim;
     double inner = o->inner_tol, last = INFINITY;
     for (int outer = 0;; ++outer) {
       if (outer > 0) {
