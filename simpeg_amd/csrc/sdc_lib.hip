@@ -260,15 +260,19 @@ struct sdc_handle_s {
   int vstore = 1;  // storage of the fp32 V-cycle vectors in this call (as sdc_params.vcycle_bf16)
   int wlevel = 0;  // level whose coarse correction runs twice (0: none)
   int wnow = 0;    // the same for the current call (solve_wlevel)
-  // single-launch coarse tail: its first level (-1: none), its descriptor, the operator image of
-  // every set (tail_img_cap floats) and the tables; tail_stale: the image does not belong to the
-  // current operator or plan (ensure_tail)
-  int tail_level = -1;
-  TailDesc tail{};
-  float *tail_img = nullptr, *tail_tab = nullptr;
-  size_t tail_img_cap = 0, tail_tab_cap = 0;
-  bool tail_stale = true;
-  bool tail_at0 = true;  // the plan may start at the finest level
+  // Single-launch coarse tail: the plans of this mesh, made once -- from the finest level on (small
+  // meshes), and from a coarser level on -- and the one of the current call (tail_of; null: none).
+  // img: the operator image of every set (img_cap floats), tab: the tables, both from the plan's
+  // first use on; stale: the image does not belong to the current operator or interpolation.
+  struct TailPlan {
+    int level = -1;  // first level (-1: no such plan)
+    TailDesc d{};
+    float *img = nullptr, *tab = nullptr;
+    size_t img_cap = 0;
+    bool stale = true;
+  };
+  TailPlan tails[2];
+  TailPlan* tail = nullptr;
   Work<float> w32;
   Work<double> w64;
   int* h_flag = nullptr;  // pinned host copy of the convergence flag
@@ -593,11 +597,14 @@ int vcycle_bytes(const sdc_handle_s* h) {
 template <typename T>
 int ensure_work(sdc_handle_s* h, int ncol) {
   Work<T>& w = work_of<T>(h);
-  const int vb = vcycle_bytes<T>(h);
-  const bool want16 =
-      std::is_same<T, float>::value && (h->vstore == 3 || h->vstore == 4);
-  if (w.ncap >= ncol && w.vbytes == vb && (w.r16 != nullptr) == want16) return SDC_OK;
+  int vb = vcycle_bytes<T>(h);
+  bool want16 = std::is_same<T, float>::value && (h->vstore == 3 || h->vstore == 4);
+  // room for wider vectors and for r16 serves narrower ones and calls without it too (the V-cycle
+  // of a Neumann handle in its bf16 storage between mixed solves in fp32)
+  if (w.ncap >= ncol && w.vbytes >= vb && (w.r16 || !want16)) return SDC_OK;
   ncol = std::max(ncol, w.ncap);
+  vb = std::max(vb, w.vbytes);
+  want16 = want16 || w.r16;
   drop_graphs(h);
   w.release();
   const int cap = std::max(ncol, 1);
@@ -689,6 +696,20 @@ int pick_wlevel(const sdc_handle_s* h) {
   return (l >= 1 && l < nl - 1) ? l : 0;
 }
 
+// The plan of a call (null: none).  Solves may run all levels of a small mesh in the tail, unless
+// the finest one reads a bf16 residual (storage 3, 4) or smooths another number of steps than the
+// coarser ones; at0 = false keeps it out as well (sdc_vcycle, whose finest level shows the storage
+// it was asked for).
+sdc_handle_s::TailPlan* tail_of(const sdc_handle_s* h, bool at0) {
+  const auto& p = h->prm;
+  if (!p.fused_tail) return nullptr;
+  if (p.vcycle_bf16 == 3 || p.vcycle_bf16 == 4) at0 = false;
+  if (p.nu_coarse > 0 && (p.nu_coarse != p.nu_pre || p.nu_coarse != p.nu_post)) at0 = false;
+  for (const auto& t : h->tails)
+    if (t.level > 0 || (t.level == 0 && at0)) return const_cast<sdc_handle_s::TailPlan*>(&t);
+  return nullptr;
+}
+
 // The same for a solve of ncol columns on a Robin operator with wcycle_level = -1.  With few
 // columns, and in fp64 on smaller meshes, the coarse levels cost the latency of their launches,
 // not bandwidth, and the second visit 20-30 % of a cycle, more than the iterations it saves, those
@@ -710,27 +731,16 @@ int solve_wlevel(const sdc_handle_s* h, int ncol, bool fp64) {
   if (h->prm.wcycle_level >= 0 || h->bc == SDC_BC_NEUMANN) return h->wlevel;
   const int w = quarter_level(h);
   if (h->L[0].nN < kWcycleNodes) return fp64 ? 0 : w;
-  const bool launched = h->tail_level < 0 || w < h->tail_level;
+  const auto* t = tail_of(h, true);
+  const bool launched = !t || w < t->level;
   return launched && (size_t)h->L[0].nN * (size_t)ncol < kWcycleColumns ? 0 : w;
 }
 
-// The coarse tail that one work-group per column runs (sdc_tail.h): from the first level with at
-// most SDC_TAIL_NODES nodes whose cycle fits into 160 KB of LDS on, with at least one level above
-// the coarsest.  The finest level may be that one, unless it reads a bf16 residual (storage 3,
-// 4) or smooths another number of steps than the coarser ones.
-// at0 = false keeps the finest level out as well (sdc_vcycle, whose finest level shows the storage
-// it was asked for).
-void pick_tail(sdc_handle_s* h, bool at0 = true) {
-  h->tail_level = -1;
-  h->tail_stale = true;
-  h->tail_at0 = at0;
+// The coarse tail that one work-group per column runs (sdc_tail.h): from the first level (from
+// `first` on) with at most SDC_TAIL_NODES nodes whose cycle fits into 160 KB of LDS on, with at
+// least one level above the coarsest.  The plan depends on the mesh alone.
+void plan_tail(const sdc_handle_s* h, sdc_handle_s::TailPlan& plan, int first) {
   const int nl = (int)h->L.size();
-  if (!h->prm.fused_tail) return;
-  const int first = !at0 || h->prm.vcycle_bf16 == 3 || h->prm.vcycle_bf16 == 4 ||
-                            (h->prm.nu_coarse > 0 && (h->prm.nu_coarse != h->prm.nu_pre ||
-                                                      h->prm.nu_coarse != h->prm.nu_post))
-                        ? 1
-                        : 0;
   for (int lt = first; lt < nl - 1; ++lt) {
     const int nlev = nl - lt;
     if (nlev > SDC_TAIL_MAX || h->L[lt].nN > SDC_TAIL_NODES) continue;
@@ -791,8 +801,8 @@ void pick_tail(sdc_handle_s* h, bool at0 = true) {
     const TailXf& x0 = d.xf[0];
     d.imgs = 8 * (size_t)tail_npt(d.lv[0].nN) * SDC_TAIL_THREADS + d.nimg +
              up4((size_t)(SDC_TAIL_WR + SDC_TAIL_WP) * x0.cN);
-    h->tail = d;
-    h->tail_level = lt;
+    plan.d = d;
+    plan.level = lt;
     return;
   }
 }
@@ -801,33 +811,28 @@ void pick_tail(sdc_handle_s* h, bool at0 = true) {
 // in Work::partial.
 template <typename T>
 uint32_t dot_blocks(const sdc_handle_s* h) {
-  return std::is_same<T, float>::value && h->tail_level == 0 ? 1u : nblk(h->L[0].nN);
+  return std::is_same<T, float>::value && h->tail && h->tail->level == 0 ? 1u : nblk(h->L[0].nN);
 }
 
-// The tail's operator image and tables on the device, for the current plan and operator sets.
+// The call's tail plan (h->tail), its operator image and tables on the device.
 int ensure_tail(sdc_handle_s* h, hipStream_t st, bool at0 = true) {
-  if (h->tail_at0 != at0) {
-    drop_graphs(h);
-    pick_tail(h, at0);
-  }
-  if (h->tail_level < 0 || !h->tail_stale) return SDC_OK;
-  const int lt = h->tail_level, nlev = (int)h->L.size() - lt;
-  TailDesc& d = h->tail;
+  h->tail = tail_of(h, at0);
+  if (!h->tail || !h->tail->stale) return SDC_OK;
+  auto& plan = *h->tail;
+  const int lt = plan.level, nlev = (int)h->L.size() - lt;
+  TailDesc& d = plan.d;
   const size_t need = d.imgs * (size_t)h->nset_cap;
   const size_t ntab = (size_t)d.ntop + d.ntab;
-  if (h->tail_img_cap < need || h->tail_tab_cap < ntab) {
+  if (plan.img_cap < need) {
     HIPCK(hipStreamSynchronize(st));
     drop_graphs(h);
-    dfree(h->tail_img);
-    dfree(h->tail_tab);
-    h->tail_img_cap = h->tail_tab_cap = 0;
-    CK(dmalloc(&h->tail_img, need));
-    CK(dmalloc(&h->tail_tab, ntab));
-    h->tail_img_cap = need;
-    h->tail_tab_cap = ntab;
-    d.tab = nullptr;
+    dfree(plan.img);
+    plan.img_cap = 0;
+    CK(dmalloc(&plan.img, need));
+    plan.img_cap = need;
   }
-  if (!d.tab) {  // a new plan (pick_tail clears d) or a new buffer
+  if (!d.tab) {
+    if (!plan.tab) CK(dmalloc(&plan.tab, ntab));
     std::vector<uint2> tab;
     for (int k = 0; k < nlev - 1; ++k) {
       const Level& f = h->L[lt + k];
@@ -852,14 +857,15 @@ int ensure_tail(sdc_handle_s* h, hipStream_t st, bool at0 = true) {
       if (k == 0) tab.resize(d.ntop / 2, uint2{0, 0});
     }
     tab.resize(ntab / 2, uint2{0, 0});
-    HIPCK(hipMemcpyAsync(h->tail_tab, tab.data(), ntab * sizeof(float), hipMemcpyHostToDevice, st));
+    HIPCK(hipMemcpyAsync(plan.tab, tab.data(), ntab * sizeof(float), hipMemcpyHostToDevice, st));
     HIPCK(hipStreamSynchronize(st));
+    d.tab = plan.tab;
   }
   TailPack p{};
   p.rows = (uint32_t)(tail_npt(d.lv[0].nN) * SDC_TAIL_THREADS);
   size_t nmax = p.rows;
   p.nlev = nlev - 1;
-  p.img = h->tail_img;
+  p.img = plan.img;
   p.imgs = d.imgs;
   const uint32_t base = 8 * p.rows;
   for (int k = 0; k < nlev - 1; ++k) {
@@ -892,18 +898,17 @@ int ensure_tail(sdc_handle_s* h, hipStream_t st, bool at0 = true) {
       if (k > 0) nmax = std::max(nmax, (size_t)w.n);
     }
   }
-  p.tab = (const uint2*)h->tail_tab;
+  p.tab = (const uint2*)plan.tab;
   p.x0 = d.xf[0];
   p.top = base + d.nimg;
   hipLaunchKernelGGL(k_tail_pack, dim3(nblk(nmax), (uint32_t)(p.nlev + 1 + p.nw - 3), (uint32_t)h->nset),
                      dim3(SDC_BLOCK), 0, st, p);
   HIPCK(hipGetLastError());
-  d.img = h->tail_img;
-  d.tab = h->tail_tab;
+  d.img = plan.img;
   d.ainv = h->ainv32;
   d.astride = (uint32_t)h->astride;
   d.nn = (int)h->L.back().nN;
-  h->tail_stale = false;
+  plan.stale = false;
   return SDC_OK;
 }
 
@@ -997,8 +1002,8 @@ Cheb cheb_coefs(const sdc_params& p) {
 // The steps of the tail's cycle: down to the W level once, its coarse correction twice (once without
 // a W level in the tail).
 void tail_program(const sdc_handle_s* h, TailDesc& d) {
-  const int w = h->wnow >= h->tail_level && h->wnow > 0 ? h->wnow - h->tail_level : -1;
-  const int last = (int)h->L.size() - 1 - h->tail_level;
+  const int w = h->wnow >= h->tail->level && h->wnow > 0 ? h->wnow - h->tail->level : -1;
+  const int last = (int)h->L.size() - 1 - h->tail->level;
   auto step = [&](TailOp op, int l) {
     d.op[d.nop] = op;
     d.lev[d.nop++] = (uint8_t)l;
@@ -1035,13 +1040,13 @@ void tail_program(const sdc_handle_s* h, TailDesc& d) {
 template <typename B, typename O>
 int tail_cycle(sdc_handle_s* h, const B* b, O* x, int ncol, double* partial, const int* done,
                hipStream_t st) {
-  if (h->tail_stale) return fail(SDC_ERR_STATE, "internal: tail image");
-  TailDesc d = h->tail;
+  if (h->tail->stale) return fail(SDC_ERR_STATE, "internal: tail image");
+  TailDesc d = h->tail->d;
   tail_program(h, d);
   d.cset = h->cur_cset;
   // level 0 smooths nu_pre / nu_post steps, coarser levels nu_coarse where that is set; a tail
-  // that holds both has one count for all its levels only if they agree (pick_tail)
-  const bool top = h->tail_level == 0 || h->prm.nu_coarse <= 0;
+  // that holds both has one count for all its levels only if they agree (tail_of)
+  const bool top = h->tail->level == 0 || h->prm.nu_coarse <= 0;
   d.nu_pre = top ? h->prm.nu_pre : h->prm.nu_coarse;
   d.nu_post = top ? h->prm.nu_post : h->prm.nu_coarse;
   d.nu_mid = h->prm.wcycle_smooth > 0 ? h->prm.wcycle_smooth : d.nu_post;
@@ -1051,7 +1056,7 @@ int tail_cycle(sdc_handle_s* h, const B* b, O* x, int ncol, double* partial, con
     d.c2[k] = (float)cc.c2[k];
   }
   const dim3 g((uint32_t)ncol), blk(SDC_TAIL_THREADS);
-  const size_t lds = (size_t)d.nlds * sizeof(float), ld = h->L[h->tail_level].ld;
+  const size_t lds = (size_t)d.nlds * sizeof(float), ld = h->L[h->tail->level].ld;
   switch (tail_npt(d.lv[0].nN)) {
     case 2: launch(h, k_tail_cycle<B, O, 2>, g, blk, lds, st, d, b, x, ld, partial, done); break;
     case 4: launch(h, k_tail_cycle<B, O, 4>, g, blk, lds, st, d, b, x, ld, partial, done); break;
@@ -1075,7 +1080,7 @@ int vcycle(sdc_handle_s* h, int l, const B* b, O* x, int ncol, bool dot_out, con
   const int nl = (int)h->L.size();
   if constexpr (std::is_same<T, float>::value &&
                 (std::is_same<B, float>::value || std::is_same<O, __bf16>::value)) {
-    if (l == h->tail_level)
+    if (h->tail && l == h->tail->level)
       return tail_cycle<B, O>(h, b, x, ncol, dot_out ? W.partial : (double*)nullptr, done, st);
   }
   if (l == nl - 1) {
@@ -1835,7 +1840,7 @@ int ensure_sets(sdc_handle_s* h, int nset) {
   }
   CK(alloc_coarse_inverse(h, nset));
   h->nset_cap = nset;
-  h->tail_stale = true;
+  for (auto& t : h->tails) t.stale = true;
   h->sigma_set = false;
   return SDC_OK;
 }
@@ -1993,7 +1998,8 @@ int sdc_create(const sdc_mesh_desc* d, sdc_handle* out) {
   }
   if (h->L.back().nN > 4096) return bail(fail(SDC_ERR_ARG, "coarsest multigrid level too large"));
   h->wlevel = pick_wlevel(h);
-  pick_tail(h);
+  plan_tail(h, h->tails[0], 0);
+  plan_tail(h, h->tails[1], 1);
   for (auto& v : h->L)
     if ((rc = alloc_level_arrays(v, 1))) return bail(rc);
   h->ncoarse = (int)h->L.back().nN;
@@ -2051,7 +2057,10 @@ int sdc_destroy(sdc_handle h) {
   dfree(h->ainv64); dfree(h->ainv32); dfree(h->gj_a); dfree(h->gj_f);
   dfree(h->tcx); dfree(h->tcy); dfree(h->tcz); dfree(h->tbd); dfree(h->trd); dfree(h->tidg);
   dfree(h->jpart);
-  dfree(h->tail_img); dfree(h->tail_tab);
+  for (auto& t : h->tails) {
+    dfree(t.img);
+    dfree(t.tab);
+  }
   dfree(h->cset_dev);
   h->w32.release();
   h->w64.release();
@@ -2104,11 +2113,12 @@ int sdc_set_params(sdc_handle h, const sdc_params* p) {
     return fail(SDC_ERR_ARG, "col_loop must be 0, 1, 8 or 16");
   DeviceGuard dg(h->device);
   drop_graphs(h);
+  if (p->interp != h->prm.interp)
+    for (auto& t : h->tails) t.stale = true;
   h->prm = *p;
   h->mixed_stalled = false;
   if (h->prm.check_every < 1) h->prm.check_every = 1;
   h->wlevel = pick_wlevel(h);
-  pick_tail(h);
   return SDC_OK;
 }
 
@@ -2216,7 +2226,7 @@ int build_levels(sdc_handle_s* h, hipStream_t st, int nset) {
 #undef SDC_CINV
   HIPCK(hipGetLastError());
   h->nset = nset;
-  h->tail_stale = true;
+  for (auto& t : h->tails) t.stale = true;
   h->sigma_set = true;
   h->mixed_stalled = false;
   return SDC_OK;
