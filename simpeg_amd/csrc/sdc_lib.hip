@@ -814,11 +814,9 @@ uint32_t dot_blocks(const sdc_handle_s* h) {
   return std::is_same<T, float>::value && h->tail && h->tail->level == 0 ? 1u : nblk(h->L[0].nN);
 }
 
-// The call's tail plan (h->tail), its operator image and tables on the device.
-int ensure_tail(sdc_handle_s* h, hipStream_t st, bool at0 = true) {
-  h->tail = tail_of(h, at0);
-  if (!h->tail || !h->tail->stale) return SDC_OK;
-  auto& plan = *h->tail;
+// A tail plan's operator image and tables on the device, for the operators that are set (or being
+// set, on st).
+int pack_tail(sdc_handle_s* h, sdc_handle_s::TailPlan& plan, hipStream_t st) {
   const int lt = plan.level, nlev = (int)h->L.size() - lt;
   TailDesc& d = plan.d;
   const size_t need = d.imgs * (size_t)h->nset_cap;
@@ -909,6 +907,20 @@ int ensure_tail(sdc_handle_s* h, hipStream_t st, bool at0 = true) {
   d.astride = (uint32_t)h->astride;
   d.nn = (int)h->L.back().nN;
   plan.stale = false;
+  return SDC_OK;
+}
+
+// The call's tail plan (h->tail), packed on its first use and after a change of the interpolation.
+// From then on whatever sets the operator packs it (build_levels), so that a recorded V-cycle runs
+// on the operator that is set when it is replayed.
+int ensure_tail(sdc_handle_s* h, hipStream_t st, bool at0 = true) {
+  h->tail = tail_of(h, at0);
+  if (!h->tail || !h->tail->stale) return SDC_OK;
+  CK(pack_tail(h, *h->tail, st));
+  // while a caller records st the image is packed when the graph runs, not yet
+  hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+  HIPCK(hipStreamIsCapturing(st, &cap));
+  h->tail->stale = cap != hipStreamCaptureStatusNone;
   return SDC_OK;
 }
 
@@ -1040,7 +1052,7 @@ void tail_program(const sdc_handle_s* h, TailDesc& d) {
 template <typename B, typename O>
 int tail_cycle(sdc_handle_s* h, const B* b, O* x, int ncol, double* partial, const int* done,
                hipStream_t st) {
-  if (h->tail->stale) return fail(SDC_ERR_STATE, "internal: tail image");
+  if (!h->tail->d.img) return fail(SDC_ERR_STATE, "internal: tail image");
   TailDesc d = h->tail->d;
   tail_program(h, d);
   d.cset = h->cur_cset;
@@ -2226,7 +2238,12 @@ int build_levels(sdc_handle_s* h, hipStream_t st, int nset) {
 #undef SDC_CINV
   HIPCK(hipGetLastError());
   h->nset = nset;
-  for (auto& t : h->tails) t.stale = true;
+  for (auto& t : h->tails) {
+    if (t.img)
+      CK(pack_tail(h, t, st));
+    else
+      t.stale = true;
+  }
   h->sigma_set = true;
   h->mixed_stalled = false;
   return SDC_OK;

@@ -68,3 +68,57 @@ def test_solves_and_cycles_in_turn(gpu, shape, bc):
         if kind == "both":
             del g
         eng.close()
+
+
+@pytest.mark.parametrize("params", [{}, {"vcycle_bf16": 0}, {"vcycle_bf16": 0, "interp": 0}])
+@pytest.mark.parametrize("shape", SHAPES)
+def test_recorded_cycle_follows_the_operator(gpu, shape, params):
+    """A recorded V-cycle runs on the operator that is set when it is replayed, and recording one
+    leaves later calls as they are, also when the operator was set between the two."""
+    eng, sig, x = _engine(shape, "Robin", seed=1, **params)
+    b = eng.to_block(x).float()
+    ref = []
+    for s in sig:
+        eng.set_sigma(s)
+        ref.append(eng.vcycle(b)[:, :eng.nN].cpu().numpy())
+    g, z = _record(eng, b)
+    for k in (0, 1, 0):
+        eng.set_sigma(sig[k])
+        g.replay()
+        assert np.array_equal(z[:, :eng.nN].cpu().numpy(), ref[k])
+        eng.set_sigma(sig[1 - k])
+        h, y = _record(eng, b)
+        assert np.array_equal(eng.vcycle(b)[:, :eng.nN].cpu().numpy(), ref[1 - k])
+        h.replay()
+        assert np.array_equal(y[:, :eng.nN].cpu().numpy(), ref[1 - k])
+        del h
+    torch.cuda.synchronize()
+    del g
+    eng.close()
+
+
+def test_recorded_cycle_beside_solves_and_sets(gpu):
+    """The same with solves and operator sets on the handle between two replays."""
+    eng, sig, x = _engine((17, 17, 17), "Robin", seed=2)
+    q = eng.to_block(np.tile(x, (1, 4))[:, :16])
+    b = q[:5].float().contiguous()
+    colset = np.repeat(np.array([0, 1], np.int32), 8)
+    eng.set_sigma_sets(sig)
+    eng.solve_sets(q, colset)
+    ref = eng.vcycle(b)[:, :eng.nN].cpu().numpy()  # set 0
+    g, z = _record(eng, b)
+    for _ in range(2):
+        eng.set_sigma(sig[1])
+        eng.solve(q, 5)
+        eng.set_params(interp=0)
+        eng.solve(q, 5)
+        eng.set_params(interp=1)
+        eng.set_sigma_sets(sig)
+        u, r = eng.solve_sets(q, colset)
+        assert r.converged
+        eng.vcycle(b)
+        g.replay()
+        assert np.array_equal(z[:, :eng.nN].cpu().numpy(), ref)
+    torch.cuda.synchronize()
+    del g
+    eng.close()
