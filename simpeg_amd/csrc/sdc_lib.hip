@@ -598,9 +598,12 @@ template <typename T>
 int ensure_work(sdc_handle_s* h, int ncol) {
   Work<T>& w = work_of<T>(h);
   int vb = vcycle_bytes<T>(h);
-  bool want16 = std::is_same<T, float>::value && (h->vstore == 3 || h->vstore == 4);
-  // room for wider vectors and for r16 serves narrower ones and calls without it too (the V-cycle
-  // of a Neumann handle in its bf16 storage between mixed solves in fp32)
+  bool want16 =
+      std::is_same<T, float>::value && (h->prm.vcycle_bf16 == 3 || h->prm.vcycle_bf16 == 4);
+  // Room for what any call with these parameters needs, so that none moves the workspace that
+  // another one (or a caller's recording of it) uses: a Neumann handle's V-cycle in its bf16
+  // storage beside mixed solves in fp32.  More room than that serves too.
+  if (std::is_same<T, float>::value && !mixed_storage(h)) vb = (int)sizeof(T);
   if (w.ncap >= ncol && w.vbytes >= vb && (w.r16 || !want16)) return SDC_OK;
   ncol = std::max(ncol, w.ncap);
   vb = std::max(vb, w.vbytes);

@@ -97,6 +97,28 @@ def test_recorded_cycle_follows_the_operator(gpu, shape, params):
     eng.close()
 
 
+@pytest.mark.parametrize("bf16", [1, 3])
+@pytest.mark.parametrize("bc", ["Robin", "Neumann"])
+def test_recorded_cycle_before_the_first_solve(gpu, bc, bf16):
+    """A solve of no more columns leaves the memory of a recorded V-cycle where it is, though it
+    keeps its vectors in another type."""
+    eng, sig, x = _engine((17, 17, 17), bc, seed=3, vcycle_bf16=bf16)
+    eng.set_sigma(sig[0])
+    q = eng.to_block(x)
+    b = q.float()
+    ref = eng.vcycle(b)[:, :eng.nN].cpu().numpy()
+    g, z = _record(eng, b)
+    hold = []
+    for _ in range(3):
+        eng.solve(q, 5)
+        hold.append(torch.full((64 << 20,), float("nan"), device=eng.device))  # what was freed
+        g.replay()
+        assert np.array_equal(z[:, :eng.nN].cpu().numpy(), ref)
+    torch.cuda.synchronize()
+    del g
+    eng.close()
+
+
 def test_recorded_cycle_beside_solves_and_sets(gpu):
     """The same with solves and operator sets on the handle between two replays."""
     eng, sig, x = _engine((17, 17, 17), "Robin", seed=2)
