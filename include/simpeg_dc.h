@@ -98,11 +98,11 @@ typedef struct {
                                   gather pass */
   int32_t wcycle_level;        /* 0: V-cycle; l >= 1: the coarse correction of level l runs twice
                                   (W-cycle on that level); -1: the first level with at most 1/4
-                                  of the finest level's nodes, but with Robin boundaries 0 in fp64
-                                  solves and sdc_vcycle on fewer than 262,144 nodes and in
-                                  solves of few columns on larger meshes.  Robin solves on the
-                                  V-cycle work towards a residual below the tolerance (tol / 10, in
-                                  fp64 tol / 32), since their errors are larger at the same one */
+                                  of the finest level's nodes, but with Robin boundaries 0 on
+                                  fewer than 262,144 nodes and in solves of few columns on
+                                  larger meshes.  Robin solves on the V-cycle work towards a
+                                  residual below the tolerance (tol / 10, in fp64 tol / 32), since
+                                  their errors are larger at the same one */
   int32_t fused_tail;          /* 1: the fp32 solver runs the small coarse levels that fit into
                                   LDS as one launch (one work-group per column); 0: off */
   int32_t refine_rhs_per_thread; /* fp64 true-residual kernel: 0 = 8, else 1, 2, 4 or 8 columns

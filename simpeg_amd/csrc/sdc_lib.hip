@@ -683,11 +683,27 @@ int quarter_level(const sdc_handle_s* h) {
   return 0;
 }
 
-// W-cycle level of the handle: the requested one, or (wcycle_level = -1) quarter_level on Neumann
-// operators and on large meshes, where a second visit there costs ~15 % of a cycle and removes
-// an iteration or two on padded meshes; elsewhere none.  Never the coarsest level.  Neumann
-// operators keep the W step: the V-cycle leaves more of the nearly free constant in the error at
-// the same residual (1.9e-9 against 1e-10 or less).
+// W-cycle level: the requested one, or (wcycle_level = -1) quarter_level on Neumann operators and on
+// large meshes, where a second visit there costs ~15 % of a cycle and removes an iteration or two
+// on padded meshes; elsewhere none.  Never the coarsest level.  Neumann operators keep the W step:
+// the V-cycle leaves more of the nearly free constant in the error at the same residual (1.9e-9
+// against 1e-10 or less).
+// On smaller Robin meshes the coarse levels cost the latency of their launches and steps, not
+// bandwidth, and the second visit 20-30 % of a cycle.  With the iterations that make up for the
+// V-cycle's errors (solve_aim) the two take about the same time on smooth models, in fp64 the V-cycle
+// less, and the W step is the weaker one on rough models: with log conductivities of standard
+// deviation 3 (correlated over 30 m) mixed solves on 22,050 and 199,080 nodes x 8 take 2.4 and
+// 10.4 ms on the V-cycle, 5.8 and 24.9 ms with the W step; white noise of standard deviation 4 on
+// 199,080 nodes converges in 0.05 s against not at all.  Time of a V-cycle solve to its aim over a W
+// one to the tolerance (random-field, block and layered models of standard deviation up to 1, means):
+//   nodes x columns    fp64   mixed          nodes x columns    fp64   mixed
+//     2,550 x  4       0.94   1.08           275,655 x  2       0.85   0.90
+//    22,050 x 20       0.90   1.03           275,655 x 24       0.93   1.02
+//    54,675 x 20       0.91   1.02           329,904 x  8       0.84   0.94
+//   106,689 x  4       0.89   0.96           329,904 x 24       0.96   1.03
+//   106,689 x 48       1.04   1.09           932,137 x  3       0.89   0.93
+//   199,080 x  4       0.85   0.91           932,137 x  8       0.97   0.97
+//   199,080 x 48       0.98   1.05         3,289,545 x  2       0.98   0.96
 constexpr uint32_t kWcycleNodes = 1u << 18;
 int pick_wlevel(const sdc_handle_s* h) {
   const int nl = (int)h->L.size();
@@ -713,30 +729,17 @@ sdc_handle_s::TailPlan* tail_of(const sdc_handle_s* h, bool at0) {
   return nullptr;
 }
 
-// The same for a solve of ncol columns on a Robin operator with wcycle_level = -1.  With few
-// columns, and in fp64 on smaller meshes, the coarse levels cost the latency of their launches,
-// not bandwidth, and the second visit 20-30 % of a cycle, more than the iterations it saves, those
-// included that make up for the V-cycle's errors (solve_aim).  Mixed solves on smaller meshes have
-// those levels in the tail, where the second visit is cheap.  Time of a V-cycle solve to its aim
-// over a W one to the tolerance (random-field, block and layered models, means):
-//   nodes x columns    fp64   mixed          nodes x columns    fp64   mixed
-//     2,550 x  4       0.94   1.08           275,655 x  2       0.85   0.90
-//    22,050 x 20       0.90   1.03           275,655 x 24       0.93   1.02
-//    54,675 x 20       0.91   1.02           329,904 x  8       0.84   0.94
-//   106,689 x  4       0.89   0.96           329,904 x 24       0.96   1.03
-//   106,689 x 48       1.04   1.09           932,137 x  3       0.89   0.93
-//   199,080 x  4       0.85   0.91           932,137 x  8       0.97   0.97
-//   199,080 x 48       0.98   1.05         3,289,545 x  2       0.98   0.96
-// (932,137 x 48 mixed, both to the tolerance: 0.98 and 1.09.)  Only where the W level runs as
-// launches.
+// The same for a solve of ncol columns: with few columns the coarse levels of a large mesh, too,
+// cost latency (the table's lower rows; 932,137 x 48, both to the tolerance: 0.98 and 1.09 on a random
+// field and a layered model).  Only where the W level runs as launches.
 constexpr size_t kWcycleColumns = (size_t)8 << 20;  // nodes x columns
-int solve_wlevel(const sdc_handle_s* h, int ncol, bool fp64) {
-  if (h->prm.wcycle_level >= 0 || h->bc == SDC_BC_NEUMANN) return h->wlevel;
-  const int w = quarter_level(h);
-  if (h->L[0].nN < kWcycleNodes) return fp64 ? 0 : w;
+int solve_wlevel(const sdc_handle_s* h, int ncol) {
   const auto* t = tail_of(h, true);
-  const bool launched = !t || w < t->level;
-  return launched && (size_t)h->L[0].nN * (size_t)ncol < kWcycleColumns ? 0 : w;
+  const bool launched = !t || h->wlevel < t->level;
+  if (h->prm.wcycle_level < 0 && h->bc != SDC_BC_NEUMANN && launched &&
+      (size_t)h->L[0].nN * (size_t)ncol < kWcycleColumns)
+    return 0;
+  return h->wlevel;
 }
 
 // The coarse tail that one work-group per column runs (sdc_tail.h): from the first level (from
@@ -2315,7 +2318,7 @@ int sdc_solve(sdc_handle h, const double* q, double* u, int ncol, const sdc_solv
     return fail(SDC_ERR_ARG, "mixed mode needs inner_tol > 0 and max_outer >= 1");
   DeviceGuard dg(h->device);
   hipStream_t st = (hipStream_t)stream;
-  h->wnow = solve_wlevel(h, ncol, o->mode == SDC_MODE_FP64);
+  h->wnow = solve_wlevel(h, ncol);
   const Level& l0 = h->L[0];
   const int R = pick_r(h, ncol, h->L[0].nN);
   const dim3 g = grid2(l0.nN, ncol, R);

@@ -1,6 +1,6 @@
 """Errors of solves at the default parameters and tolerance against those with the W step on the
-first level of at most a quarter of the nodes, on Robin meshes where the automatic cycle can be the V-cycle (fp64 below 262,144 nodes, and few
-columns on a larger mesh): the V-cycle leaves more of the smooth error at the same residual, so its solves
+first level of at most a quarter of the nodes, on Robin meshes where the automatic cycle can be the V-cycle (below 262,144 nodes, and few columns
+on a larger mesh): the V-cycle leaves more of the smooth error at the same residual, so its solves
 have to work towards a smaller one.  A single pair depends on where the last iteration lands, so
 the geometric mean over the models and columns is compared."""
 
@@ -41,3 +41,26 @@ def test_errors_not_above_those_of_the_w_cycle(gpu, mode, core, npad, columns, w
             ratio.append(err[-1] / err[wlevel])
     print(mode, core, ["%.2f" % v for v in ratio])
     assert np.exp(np.mean(np.log(ratio))) <= 1.0
+
+
+@pytest.mark.parametrize("core,npad,std,columns", [((24, 24, 12), 5, 4.0, 8),
+                                                   ((64, 48, 32), 7, 4.0, 8)])
+def test_rough_models(gpu, core, npad, std, columns):
+    """White noise of standard deviation 4 in the log conductivity: default mixed solves converge
+    within the default iteration limit and agree with fp64 ones (which the W-cycle does not
+    reach on the larger mesh)."""
+    from simpeg_amd import maps, workloads as W
+    from simpeg_amd.resistivity import Simulation3DNodal
+
+    mesh = W.padded_mesh(core, npad=npad)
+    survey = W.grid_survey(2, 4, 2, spacing=10.0, y_span=100.0)
+    sim = Simulation3DNodal(mesh, survey=survey, sigmaMap=maps.ExpMap(mesh))
+    eng = sim.engine
+    eng.set_sigma(0.01 * np.exp(std * np.random.default_rng(1).standard_normal(eng.nC)))
+    q = sim._source_block()[:columns].contiguous()
+    u, res = eng.solve(q, columns)
+    assert res.converged and res.max_rel_res <= 1e-10, res
+    ref, _ = eng.solve(q, columns, mode="fp64", tol=1e-12)
+    d = (u - ref)[:columns, :eng.nN].norm(dim=1) / ref[:columns, :eng.nN].norm(dim=1)
+    print(res, float(d.max()))
+    assert float(d.max()) < 1e-6  # a contrast of e^30 amplifies the residual
