@@ -1354,11 +1354,18 @@ __global__ __launch_bounds__(SDC_FIN_THREADS) void k_norm_decide(const double* _
 // previous update than 2^-SDC_STALL_RATE per iteration (the caller continues in fp64).  At the
 // stop the control block is also written to hctl (pinned host memory, may be null) for the host
 // to read, and every update leaves a note there (sequence number 2 it + 1).
-// The rate: an fp64 iteration costs 2.5-3 mixed ones and gains about 2.8 octaves of residual
-// (10 decades in 12 iterations), so a mixed phase below a quarter of that is slower than fp64.
-// Ordinary models gain 2.2 to 3.7 octaves per mixed iteration, a block of contrast 1e3 1.5, one
-// of 1e4 0.2 (174 iterations on 2,550 nodes without this rule, 32 + 7 fp64 ones with it).
-#define SDC_STALL_RATE 0.66
+// The rate: an fp64 iteration costs 1.6 (few columns) to 2.7 mixed ones (many) and gains about 2.8
+// octaves of residual on ordinary models (10 decades in 12 iterations), but 0.4 to 1 on rough ones,
+// where the mixed iteration gains about as much and must go on.  Ordinary models gain 2.2 to 3.7
+// octaves per mixed iteration, a block of contrast 1e3 1.5, one of 1e4 0.2 to 0.5 after a fast start
+// (174 iterations on 2,550 nodes without this rule).  Rates of 0.66, 0.45 and 0.33, ms per first
+// solve of 48 columns (and of a later one, which runs in fp64 if the first gave up):
+//   30 % of the cells 1e3 times as conductive: 199,080 nodes 31 (38), 17, 17; 462,840 79 (93), 35, 35
+//   white noise, standard deviation 2 and 3, 199,080: 23 (25), 14, 14 and 53 (54), 53 (54), 30
+//   a block of contrast 1e4: 199,080 15 (13), 18 (13), 18 (13); 462,840 30 (28), 35 (28), 37 (37)
+// A quarter of the best rate of the solve so far in its place was no better a judge: rough models
+// start fast, too.
+#define SDC_STALL_RATE 0.33
 __global__ __launch_bounds__(SDC_FIN_THREADS) void k_true_after(const double* __restrict__ partial,
                                                                 uint32_t nbx,
                                                                 const double* __restrict__ qn2,
