@@ -94,7 +94,8 @@ typedef struct {
                                   reads a bfloat16 copy of the residual; 4: as 1, and the finest
                                   level reads a bfloat16 copy of the residual; 0: fp32 vectors.
                                   Mixed solves of Neumann operators always use fp32 vectors */
-  int32_t xfer_separable;      /* restriction: 1 = one pass per coarsened axis, 0 = one 27-point
+  int32_t xfer_separable;      /* restriction: 1 = factor by factor (x with the residual, y and z
+                                  in one pass, where these axes are coarsened), 0 = one 27-point
                                   gather pass */
   int32_t wcycle_level;        /* 0: V-cycle; l >= 1: the coarse correction of level l runs twice
                                   (W-cycle on that level); -1: the first level with at most 1/4

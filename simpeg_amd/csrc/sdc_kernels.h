@@ -1147,8 +1147,8 @@ __global__ __launch_bounds__(SDC_BLOCK) void k_update_r4(float* __restrict__ r,
 // asks for a fold (reliable update or full ring).  UFRESH: u holds nothing yet (first fold of a
 // solve): u = the sum without reading u, and the column padding [nN, ld) is zeroed, so the
 // solve needs no separate clearing pass.  u comes from the pointer table (u = qu[1]); a
-// work-group covers SDC_FOLD_CHUNKS chunks of SDC_NODES4 nodes (most launches only read the
-// flags and return).
+// work-group covers SDC_FOLD_CHUNKS chunks of SDC_NODES4 nodes (with check_every > 1 most launches
+// only read the flags and return).
 __global__ __launch_bounds__(SDC_BLOCK) void k_ir_fold_ring(const double* const* qu,
                                                             const float* const* ptab,
                                                             const double* __restrict__ ahist,

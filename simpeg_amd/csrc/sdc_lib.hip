@@ -684,19 +684,20 @@ int quarter_level(const sdc_handle_s* h) {
   return 0;
 }
 
-// W-cycle level: the requested one, or (wcycle_level = -1) quarter_level on Neumann operators and on
-// large meshes, where a second visit there costs ~15 % of a cycle and removes an iteration or two
-// on padded meshes; elsewhere none.  Never the coarsest level.  Neumann operators keep the W step:
-// the V-cycle leaves more of the nearly free constant in the error at the same residual (1.9e-9
-// against 1e-10 or less).
+// W-cycle level: the requested one, or (wcycle_level = -1) quarter_level on Neumann operators and
+// on large meshes, where a second visit there costs ~15 % of a cycle and removes an iteration or
+// two on padded meshes; elsewhere none.  Never the coarsest level.  Neumann operators keep the W
+// step: the V-cycle leaves more of the nearly free constant in the error at the same residual
+// (1.9e-9 against 1e-10 or less).
 // On smaller Robin meshes the coarse levels cost the latency of their launches and steps, not
 // bandwidth, and the second visit 20-30 % of a cycle.  With the iterations that make up for the
-// V-cycle's errors (solve_aim) the two take about the same time on smooth models, in fp64 the V-cycle
-// less, and the W step is the weaker one on rough models: with log conductivities of standard
-// deviation 3 (correlated over 30 m) mixed solves on 22,050 and 199,080 nodes x 8 take 2.4 and
-// 10.4 ms on the V-cycle, 5.8 and 24.9 ms with the W step; white noise of standard deviation 4 on
-// 199,080 nodes converges in 0.05 s against not at all.  Time of a V-cycle solve to its aim over a W
-// one to the tolerance (random-field, block and layered models of standard deviation up to 1, means):
+// V-cycle's errors (solve_aim) the two take about the same time on smooth models, in fp64 the
+// V-cycle less, and the W step is the weaker one on rough models: with log conductivities of
+// standard deviation 3 (correlated over 30 m) mixed solves on 22,050 and 199,080 nodes x 8 take
+// 2.6 and 11.0 ms on the V-cycle, 5.8 and 24.9 ms with the W step; white noise of standard
+// deviation 4 on 199,080 nodes converges in 0.05 s against not at all.  Time of a V-cycle solve to
+// its aim over a W one to the tolerance (means over random-field, block and layered models of
+// standard deviation up to 1):
 //   nodes x columns    fp64   mixed          nodes x columns    fp64   mixed
 //     2,550 x  4       0.94   1.08           275,655 x  2       0.85   0.90
 //    22,050 x 20       0.90   1.03           275,655 x 24       0.93   1.02
@@ -731,8 +732,8 @@ sdc_handle_s::TailPlan* tail_of(const sdc_handle_s* h, bool at0) {
 }
 
 // The same for a solve of ncol columns: with few columns the coarse levels of a large mesh, too,
-// cost latency (the table's lower rows; 932,137 x 48, both to the tolerance: 0.98 and 1.09 on a random
-// field and a layered model).  Only where the W level runs as launches.
+// cost latency (the table's right half; 932,137 x 48, both to the tolerance: 0.98 and 1.09 on a
+// random field and a layered model).  Only where the W level runs as launches.
 constexpr size_t kWcycleColumns = (size_t)8 << 20;  // nodes x columns
 int solve_wlevel(const sdc_handle_s* h, int ncol) {
   const auto* t = tail_of(h, true);
@@ -1018,8 +1019,8 @@ Cheb cheb_coefs(const sdc_params& p) {
   return c;
 }
 
-// The steps of the tail's cycle: down to the W level once, its coarse correction twice (once without
-// a W level in the tail).
+// The steps of the tail's cycle: down to the W level once, its coarse correction twice (once
+// without a W level in the tail).
 void tail_program(const sdc_handle_s* h, TailDesc& d) {
   const int w = h->wnow >= h->tail->level && h->wnow > 0 ? h->wnow - h->tail->level : -1;
   const int last = (int)h->L.size() - 1 - h->tail->level;
@@ -1405,9 +1406,9 @@ int graph_run(sdc_handle_s* h, const void* b, void* x, int ncol, int variant, hi
 // Wait until the solve's note to the host has reached sequence number `seq` and return it.  The
 // host reads the word itself for a while: a stream synchronisation returns some 10 us after the
 // kernel that wrote the note, as long as three kernels of a small problem take.  Between the reads
-// it lets other threads run, which may have solves of their own to launch (eight problems on eight
-// threads: 9.7 ms on one CPU without that, 6.2 with it; 9.5 and 6.8 on four).  Past kNoteSpin (large
-// problems, where it does not matter) it gives the CPU back and synchronises.
+// it lets other threads run, which may have solves of their own to launch (eight problems on
+// eight threads: 9.6 ms on one CPU without that, 6.1 with it; 8.4 and 7.5 on four).  Past kNoteSpin
+// (large problems, where it does not matter) it gives the CPU back and synchronises.
 int wait_note(sdc_handle_s* h, hipStream_t st, int seq, int* note) {
   constexpr auto kNoteSpin = std::chrono::microseconds(500);
   const int* p = (const int*)h->h_ctl + SDC_CTL_NOTE;
@@ -1533,15 +1534,15 @@ int pcg(sdc_handle_s* h, T* x, int ncol, double tol, int maxit, const int* col_m
 // the residual.  A solve that ends between the two still has converged, and none is asked for less
 // than the sums of its precision can show.
 // Neumann operators, mixed: nothing but the three edges of the grounded corner holds the constant,
-// so a residual's sum shifts all potentials: at 22,000..230,000 nodes (20 solves) the error of u was
-// up to 107 times the relative residual (8.5e-9 at 7.9e-11).  Two iterations more of 10 to 15 take it
-// to 1.5e-10 at the default tolerance.
+// so a residual's sum shifts all potentials: at 22,000..230,000 nodes (20 solves) the error of u
+// was up to 107 times the relative residual (8.5e-9 at 7.9e-11).  Two iterations more of 10 to 15
+// take it to 1.5e-10 at the default tolerance.
 // Robin operators, V-cycle where the mesh has a level for the W step: at the same residual the
-// V-cycle leaves more of the smooth error, and its last iteration passes the tolerance by less.  Over
-// 117 problems (2,550..3,289,545 nodes, 1..48 columns, three kinds of model) the errors of V-cycle
-// solves to the tolerance were 1.3 to 19 times those of W-cycle solves in fp64 (mean per size; at
-// most 115) and 0.6 to 12 times in mixed precision; to the aims here 0.04 to 0.45 (at most 2.7) and
-// 0.08 to 0.64 times.
+// V-cycle leaves more of the smooth error, and its last iteration passes the tolerance by less.
+// Over 117 problems (2,550..3,289,545 nodes, 1..48 columns, three kinds of model) the errors of
+// V-cycle solves to the tolerance were 1.3 to 19 times those of W-cycle solves in fp64 (means per
+// size; at most 115) and 0.6 to 12 times in mixed precision; to the aims here 0.04 to 0.45 (at most
+// 2.7) and 0.08 to 0.64 times.
 double solve_aim(const sdc_handle_s* h, double tol, bool fp64) {
   double f = 1.0;
   if (h->bc == SDC_BC_NEUMANN)
@@ -1556,9 +1557,11 @@ double solve_aim(const sdc_handle_s* h, double tol, bool fp64) {
 // column's fp32 residual passed the tolerance, or some column's residual dropped by
 // reliable_delta since its last replacement.  Columns stop on the true residual only.
 // Every decision is taken on the device (k_norm_decide, k_true_after on the control block
-// W.ctl): an iteration is a fixed sequence of launches whose kernels return at once when the
-// control block says the solve stopped or no update is due, so check_every iterations at a time
-// run without a host synchronisation -- as one recorded graph when sdc_params.graph is set.
+// W.ctl).  With check_every = 1 the host reads it as a note and launches the fold, the fp64 residual
+// and the stop test only when they are due; with more, an iteration is a fixed sequence of
+// launches whose kernels return at once when the control block says the solve stopped or no update
+// is due, so check_every iterations run without a host synchronisation.  Iterations are recorded
+// graphs when sdc_params.graph is set.
 int pcg_reliable(sdc_handle_s* h, const double* q, double* u, int ncol, const sdc_solve_opts* o,
                  sdc_solve_stats& S, hipStream_t st) {
   h->vstore = mixed_storage(h);
@@ -1571,10 +1574,10 @@ int pcg_reliable(sdc_handle_s* h, const double* q, double* u, int ncol, const sd
   const dim3 g = grid2(l0.nN, ncol, R);
   const dim3 blk(SDC_BLOCK);
   const uint32_t nbx = nblk(l0.nN);
-  // 4 node blocks per work-group of the fp64 residual: its empty launches (no reliable update)
-  // are cheap (cfg 2: 9.7 us).  With 8 its full pass took 686-702 against 705-733 us but
-  // fetched 3.84 against 2.77 GB from HBM (5.5 TB/s), too close to the bandwidth that
-  // concurrent streams share.
+  // 4 node blocks per work-group of the fp64 residual: a quarter of the partials for k_true_after,
+  // and with check_every > 1 cheap empty launches (932,137 nodes x 128 columns: 9.7 us).  With 8 the
+  // pass took 686-702 against 705-733 us but fetched 3.84 against 2.77 GB from HBM (5.5 TB/s), too
+  // close to the bandwidth that concurrent streams share.
   constexpr int kIrChunks = 4;
   const uint32_t nbx_ir = (nbx + kIrChunks - 1) / kIrChunks;
   // r update: kUpdChunks chunks of SDC_NODES4 nodes per work-group, so that k_norm_decide sums
@@ -1742,8 +1745,8 @@ int pcg_reliable(sdc_handle_s* h, const double* q, double* u, int ncol, const sd
            (const int*)W.active, ncol, S_, notes ? h->d_ctl : nullptr);
     return SDC_OK;
   };
-  // Reliable update or fold (every kernel returns at once unless k_norm_decide asked for it);
-  // for profiled runs: fresh, u has not been written yet; pend, the directions folded
+  // Reliable update or fold (launched when it is due, or, with check_every > 1, always: every kernel
+  // returns at once unless k_norm_decide asked for it); for profiled runs: fresh, u has not been written yet; pend, the directions folded
   auto update = [&](hipStream_t s, int it, bool upd, bool fresh, int pend) -> int {
     const int phi = it % S_;
     prof_begin(h, SDC_PROF_FOLD, s);
@@ -1754,7 +1757,7 @@ int pcg_reliable(sdc_handle_s* h, const double* q, double* u, int ncol, const sd
     // algorithmic bytes: the pending directions read, u read (unless fresh) and written
     prof_end(h, SDC_PROF_FOLD, s, (double)l0.nN * ncol * (4.0 * pend + (fresh ? 8 : 16)));
     prof_begin(h, upd ? SDC_PROF_REFINE : -1, s);
-    // kIrChunks node blocks per work-group: most launches return at once (no update)
+    // kIrChunks node blocks per work-group
     DISPATCH_RG(R64, G_, launch(h, (k_ir_residual<float, R, false, G, kIrChunks>),
                                 dim3(nbx_ir, (uint32_t)((ncol + R * G - 1) / (R * G))), blk, 0,
                                 s, s2, (const double*)nullptr, (const double*)nullptr, W.r,

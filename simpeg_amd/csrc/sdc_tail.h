@@ -11,14 +11,15 @@
 //
 // What bounds it is latency: a step is a few hundred LDS reads per wave between two barriers, so
 // no step may wait for L2.  The top level's coefficients stay in registers from the first step to
-// the last (up to 8 nodes a work-item; 1,024 work-items fill the register file at 128 each), with
-// the rows scaled by the inverse diagonal: six weights, A' x = x - sum w x_nbr.  Its iterate is
-// the only top-level vector in LDS.  The lower levels' scaled coefficients, their interpolation
+// the last (up to 8 nodes a work-item; 1,024 work-items fill the register file at 128 each, and the
+// form of 8 nodes, for top levels of more than 4,096, is over it by 6 to 16 registers that live
+// in scratch memory), with the rows scaled by the inverse diagonal: six weights,
+// A' x = x - sum w x_nbr.  Its iterate is the only top-level vector in LDS.  The lower levels' scaled coefficients, their interpolation
 // weights and the transfers' tables come into LDS with one copy of an image that k_tail_pack lays
 // out when the operator is set.  With the coefficients read from L2 in every step (the form
-// before) the levels of 7,406 + 1,352 + 245 + 48 nodes took 59-86 us per launch, now 33; of that
-// 5 us load the 350 KB of image and coefficients, 2-3 us go to each step of the top level and
-// 1-2 us to each step of a lower one.
+// before) the levels of 7,406 + 1,352 + 245 + 48 nodes took 59-86 us per launch, now 33 (3 columns)
+// to 38 (128); of that 5 us load the 350 KB of image and coefficients, 2-3 us go to each step of
+// the top level and 1-2 us to each step of a lower one.
 #pragma once
 #include "sdc_kernels.h"
 
@@ -39,9 +40,10 @@ struct TailLev {
 // Transfer between level l and l + 1: strides of the grids, the LDS offset of its table (two
 // words per coarse node, tail_table_entry; the top level's is read from global memory) and where
 // its interpolation weights start (Xfer::wx, wy, wz one after the other): LDS offset w.  The top
-// level's weights are laid out per coarse node in the image instead (SDC_TAIL_WR for the restriction, SDC_TAIL_WP for the interpolation, each
-// an array over the coarse nodes): read from L2 point by point, 9 gathers of stride 2 per
-// work-item, they took 20,000 of a launch's 77,000 clocks on 7,406 + 1,352 nodes.
+// level's weights are laid out per coarse node in the image instead (SDC_TAIL_WR for the
+// restriction, SDC_TAIL_WP for the interpolation, each an array over the coarse nodes): read from
+// L2 point by point, 9 gathers of stride 2 per work-item, they took 20,000 of a launch's 77,000
+// clocks on 7,406 + 1,352 nodes.
 #define SDC_TAIL_WR 27
 #define SDC_TAIL_WP 12
 struct TailXf {
@@ -404,7 +406,7 @@ __global__ __launch_bounds__(SDC_TAIL_THREADS) void k_tail_cycle(TailDesc d,
       const float* xn = X + tid + k * NT;
       t[k] = bs[k] - xn[0] + wxm[k] * xn[-1] + wxp[k] * xn[1] + wym[k] * xn[-n1] +
              wyp[k] * xn[n1] + wzm[k] * xn[-pl] + wzp[k] * xn[pl];
-      // at most two nodes' reads in flight: all 56 at once spilled the weights
+      // at most two nodes' reads in flight: all 56 at once moved the weights to scratch memory
       if (k & 1) asm volatile("" ::: "memory");
     }
   };
