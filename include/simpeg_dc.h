@@ -102,8 +102,8 @@ typedef struct {
                                   of the finest level's nodes, but with Robin boundaries 0 on
                                   fewer than 262,144 nodes and in solves of few columns on
                                   larger meshes.  Robin solves on the V-cycle work towards a
-                                  residual below the tolerance (tol / 10, in fp64 tol / 32), since
-                                  their errors are larger at the same one */
+                                  residual below the tolerance (tol / 4 to tol / 32), since their
+                                  errors are larger at the same one */
   int32_t fused_tail;          /* 1: the fp32 solver runs the small coarse levels that fit into
                                   LDS as one launch (one work-group per column); 0: off */
   int32_t refine_rhs_per_thread; /* fp64 true-residual kernel: 0 = 8, else 1, 2, 4 or 8 columns

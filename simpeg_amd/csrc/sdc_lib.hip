@@ -699,9 +699,9 @@ int quarter_level(const sdc_handle_s* h) {
 // its aim over a W one to the tolerance (means over random-field, block and layered models of
 // standard deviation up to 1):
 //   nodes x columns    fp64   mixed          nodes x columns    fp64   mixed
-//     2,550 x  4       0.94   1.08           275,655 x  2       0.85   0.90
-//    22,050 x 20       0.90   1.03           275,655 x 24       0.93   1.02
-//    54,675 x 20       0.91   1.02           329,904 x  8       0.84   0.94
+//     2,550 x  4       0.91   1.05           275,655 x  2       0.85   0.90
+//    22,050 x 20       0.86   1.00           275,655 x 24       0.93   1.02
+//    54,675 x 20       0.86   0.98           329,904 x  8       0.84   0.94
 //   106,689 x  4       0.89   0.96           329,904 x 24       0.96   1.03
 //   106,689 x 48       1.04   1.09           932,137 x  3       0.89   0.93
 //   199,080 x  4       0.85   0.91           932,137 x  8       0.97   0.97
@@ -1539,16 +1539,20 @@ int pcg(sdc_handle_s* h, T* x, int ncol, double tol, int maxit, const int* col_m
 // take it to 1.5e-10 at the default tolerance.
 // Robin operators, V-cycle where the mesh has a level for the W step: at the same residual the
 // V-cycle leaves more of the smooth error, and its last iteration passes the tolerance by less.
-// Over 117 problems (2,550..3,289,545 nodes, 1..48 columns, three kinds of model) the errors of
-// V-cycle solves to the tolerance were 1.3 to 19 times those of W-cycle solves in fp64 (means per
-// size; at most 115) and 0.6 to 12 times in mixed precision; to the aims here 0.04 to 0.45 (at most
-// 2.7) and 0.08 to 0.64 times.
+// Errors of V-cycle solves over those of W-cycle solves (both stop at their residual; means per size
+// and column count over 213 problems of 1..48 columns and three kinds of model, in brackets the
+// largest single ratio), for V-cycle residuals of the tolerance and of the aim:
+//   nodes                      fp64: tol       aim             mixed: tol      aim
+//   2,550..54,675              1.2..2.9 (19)   0.11..0.24 (2)  0.6..1.6 (11)   0.22..0.46 (4)
+//   68,355..329,904            1.6..13 (85)    0.06..0.40 (3)  1.1..12 (48)    0.12..0.64 (12)
+//   932,137 and 3,289,545      6..19 (115)     0.24..0.45 (2)  3..7 (40)       0.35..0.58 (3)
+constexpr uint32_t kAimNodes = 1u << 16;
 double solve_aim(const sdc_handle_s* h, double tol, bool fp64) {
   double f = 1.0;
   if (h->bc == SDC_BC_NEUMANN)
     f = fp64 ? 1.0 : 32.0;
   else if (h->wnow == 0 && quarter_level(h) > 0)
-    f = fp64 ? 32.0 : 10.0;
+    f = h->L[0].nN < kAimNodes ? (fp64 ? 10.0 : 4.0) : (fp64 ? 32.0 : 10.0);
   return std::min(tol, std::max(tol / f, fp64 ? 1e-14 : 2e-12));
 }
 
