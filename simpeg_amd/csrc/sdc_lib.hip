@@ -833,6 +833,7 @@ int pack_tail(sdc_handle_s* h, sdc_handle_s::TailPlan& plan, hipStream_t st) {
     HIPCK(hipStreamSynchronize(st));
     drop_graphs(h);
     dfree(plan.img);
+    d.img = nullptr;
     plan.img_cap = 0;
     CK(dmalloc(&plan.img, need));
     plan.img_cap = need;
