@@ -1540,9 +1540,9 @@ int pcg(sdc_handle_s* h, T* x, int ncol, double tol, int maxit, const int* col_m
 // take it to 1.5e-10 at the default tolerance.
 // Robin operators, V-cycle where the mesh has a level for the W step: at the same residual the
 // V-cycle leaves more of the smooth error, and its last iteration passes the tolerance by less.
-// Errors of V-cycle solves over those of W-cycle solves (both stop at their residual; means per size
-// and column count over 213 problems of 1..48 columns and three kinds of model, in brackets the
-// largest single ratio), for V-cycle residuals of the tolerance and of the aim:
+// Errors of V-cycle solves over those of W-cycle solves to the tolerance (means per size and column
+// count over 213 problems of 1..48 columns and three kinds of model, in brackets the largest single
+// ratio), for V-cycle solves to the tolerance and to the aim:
 //   nodes                      fp64: tol       aim             mixed: tol      aim
 //   2,550..54,675              1.2..2.9 (19)   0.11..0.24 (2)  0.6..1.6 (11)   0.22..0.46 (4)
 //   68,355..329,904            1.6..13 (85)    0.06..0.40 (3)  1.1..12 (48)    0.12..0.64 (12)
@@ -1562,11 +1562,11 @@ double solve_aim(const sdc_handle_s* h, double tol, bool fp64) {
 // column's fp32 residual passed the tolerance, or some column's residual dropped by
 // reliable_delta since its last replacement.  Columns stop on the true residual only.
 // Every decision is taken on the device (k_norm_decide, k_true_after on the control block
-// W.ctl).  With check_every = 1 the host reads it as a note and launches the fold, the fp64 residual
-// and the stop test only when they are due; with more, an iteration is a fixed sequence of
-// launches whose kernels return at once when the control block says the solve stopped or no update
-// is due, so check_every iterations run without a host synchronisation.  Iterations are recorded
-// graphs when sdc_params.graph is set.
+// W.ctl).  With check_every = 1 the host reads it as a note and launches the fold, the fp64
+// residual and the stop test only when they are due; with more, an iteration is a fixed sequence
+// of launches whose kernels return at once when the control block says the solve stopped or no
+// update is due, so check_every iterations run without a host synchronisation.  Iterations are
+// recorded graphs when sdc_params.graph is set.
 int pcg_reliable(sdc_handle_s* h, const double* q, double* u, int ncol, const sdc_solve_opts* o,
                  sdc_solve_stats& S, hipStream_t st) {
   h->vstore = mixed_storage(h);
@@ -1750,8 +1750,9 @@ int pcg_reliable(sdc_handle_s* h, const double* q, double* u, int ncol, const sd
            (const int*)W.active, ncol, S_, notes ? h->d_ctl : nullptr);
     return SDC_OK;
   };
-  // Reliable update or fold (launched when it is due, or, with check_every > 1, always: every kernel
-  // returns at once unless k_norm_decide asked for it); for profiled runs: fresh, u has not been written yet; pend, the directions folded
+  // Reliable update or fold (launched when it is due, or, with check_every > 1, always: every
+  // kernel returns at once unless k_norm_decide asked for it); for profiled runs: fresh, u has not
+  // been written yet; pend, the directions folded
   auto update = [&](hipStream_t s, int it, bool upd, bool fresh, int pend) -> int {
     const int phi = it % S_;
     prof_begin(h, SDC_PROF_FOLD, s);
