@@ -1357,8 +1357,8 @@ __global__ __launch_bounds__(SDC_FIN_THREADS) void k_norm_decide(const double* _
 // The rate: an fp64 iteration costs 1.6 (few columns) to 2.7 mixed ones (many) and gains about 2.8
 // octaves of residual on ordinary models (10 decades in 12 iterations), but 0.4 to 1 on rough ones,
 // where the mixed iteration gains about as much and must go on.  Ordinary models gain 2.2 to 3.7
-// octaves per mixed iteration, a block of contrast 1e3 1.5, one of 1e4 0.2 to 0.5 after a fast start
-// (174 iterations on 2,550 nodes without this rule).  Rates of 0.66, 0.45 and 0.33, ms per first
+// octaves per mixed iteration, a block of contrast 1e3 1.5, one of 1e4 0.2 to 0.5 after a fast
+// start (174 iterations on 2,550 nodes without this rule).  Rates of 0.66, 0.45 and 0.33, ms per first
 // solve of 48 columns (and of a later one, which runs in fp64 if the first gave up):
 //   30 % of the cells 1e3 times as conductive: 199,080 nodes 31 (38), 17, 17; 462,840 79 (93), 35, 35
 //   white noise, standard deviation 2 and 3, 199,080: 23 (25), 14, 14 and 53 (54), 53 (54), 30

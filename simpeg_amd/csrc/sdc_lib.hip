@@ -1541,7 +1541,7 @@ int pcg(sdc_handle_s* h, T* x, int ncol, double tol, int maxit, const int* col_m
 // Robin operators, V-cycle where the mesh has a level for the W step: at the same residual the
 // V-cycle leaves more of the smooth error, and its last iteration passes the tolerance by less.
 // Errors of V-cycle solves over those of W-cycle solves to the tolerance (means per size and column
-// count over 213 problems of 1..48 columns and three kinds of model, in brackets the largest single
+// count over 252 problems of 1..48 columns and three kinds of model, in brackets the largest single
 // ratio), for V-cycle solves to the tolerance and to the aim:
 //   nodes                      fp64: tol       aim             mixed: tol      aim
 //   2,550..54,675              1.2..2.9 (19)   0.11..0.24 (2)  0.6..1.6 (11)   0.22..0.46 (4)

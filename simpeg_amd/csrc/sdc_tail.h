@@ -14,9 +14,9 @@
 // the last (up to 8 nodes a work-item; 1,024 work-items fill the register file at 128 each, and the
 // form of 8 nodes, for top levels of more than 4,096, is over it by 6 to 16 registers that live
 // in scratch memory), with the rows scaled by the inverse diagonal: six weights,
-// A' x = x - sum w x_nbr.  Its iterate is the only top-level vector in LDS.  The lower levels' scaled coefficients, their interpolation
-// weights and the transfers' tables come into LDS with one copy of an image that k_tail_pack lays
-// out when the operator is set.  With the coefficients read from L2 in every step (the form
+// A' x = x - sum w x_nbr.  Its iterate is the only top-level vector in LDS.  The lower levels'
+// scaled coefficients, their interpolation weights and the transfers' tables come into LDS with
+// one copy of an image that k_tail_pack lays out when the operator is set.  With the coefficients read from L2 in every step (the form
 // before) the levels of 7,406 + 1,352 + 245 + 48 nodes took 59-86 us per launch, now 33 (3 columns)
 // to 38 (128); of that 5 us load the 350 KB of image and coefficients, 2-3 us go to each step of
 // the top level and 1-2 us to each step of a lower one.

@@ -1,8 +1,9 @@
 """Errors of solves at the default parameters and tolerance against those with the W step on the
-first level of at most a quarter of the nodes, on Robin meshes where the automatic cycle can be the V-cycle (below 262,144 nodes, and few columns
-on a larger mesh): the V-cycle leaves more of the smooth error at the same residual, so its solves
-have to work towards a smaller one.  A single pair depends on where the last iteration lands, so
-the geometric mean over the models and columns is compared."""
+first level of at most a quarter of the nodes, on Robin meshes where the automatic cycle can be
+the V-cycle (below 262,144 nodes, and few columns on a larger mesh): the V-cycle leaves more of
+the smooth error at the same residual, so its solves have to work towards a smaller one.  A single
+pair depends on where the last iteration lands, so the geometric mean over the models and columns
+is compared."""
 
 import numpy as np
 import pytest
